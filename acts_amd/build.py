@@ -8,15 +8,22 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 REPO_DIR = os.path.dirname(PKG_DIR)
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_PATH = os.path.join(PKG_DIR, "libacts_kf.so")
 
-SOURCES = ["kf_capi.hip", "generator.hip"]
+# (source, defines) of every object of the library; the forward kernel's
+# variants are compiled one by one
+OBJECTS = [("kf_capi.hip", []), ("generator.hip", [])] + [
+    ("kf_forward.hip", [f"-DKF_MIXED={m}", f"-DKF_SYMPY={s}", f"-DKF_LAYERS={n}"])
+    for m in (0, 1) for s in (0, 1) for n in (0, 1)]
 HEADERS = ["kf_common.hpp", "kf_device.hpp", "kf_mixed.hpp", "kf_fit.hpp", "kf_kernel.hpp",
-           "kf_reference.hpp", "kf_reverse.hpp", "kf_states.hpp", "kf_field_host.hpp"]
+           "kf_reference.hpp", "kf_reverse.hpp", "kf_forward.hpp", "kf_states.hpp",
+           "kf_field_host.hpp"]
 
 # -ffp-contract=off: the FP64 fit keeps the reference's separate multiply and
 # add roundings (x86-64 without -march has no FMA), so every decision of the
@@ -26,7 +33,6 @@ HIPCC_FLAGS = [
     "-O3",
     "-std=c++17",
     "-fPIC",
-    "-shared",
     "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
@@ -42,16 +48,25 @@ def hipcc_path() -> str:
 
 def build_library(verbose: bool = False, extra_flags: list[str] | None = None) -> str:
     """Compile libacts_kf.so in-tree; returns its path."""
-    srcs = [os.path.join(CSRC, s) for s in SOURCES]
     tmp = LIB_PATH + ".tmp"
-    cmd = [hipcc_path(), *HIPCC_FLAGS, *(extra_flags or []), "-o", tmp, *srcs,
-           "-lpthread"]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        sys.stderr.write(res.stdout + res.stderr)
-        raise RuntimeError("hipcc failed building libacts_kf.so")
+    flags = [*HIPCC_FLAGS, *(extra_flags or [])]
+
+    def run(cmd):
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        res = subprocess.run(cmd, capture_output=True, text=True)
+        if res.returncode != 0:
+            sys.stderr.write(res.stdout + res.stderr)
+            raise RuntimeError("hipcc failed building libacts_kf.so")
+
+    with tempfile.TemporaryDirectory() as work:
+        objs = [os.path.join(work, f"{i}.o") for i in range(len(OBJECTS))]
+        jobs = [[hipcc_path(), *flags, *defines, "-c", "-o", obj, os.path.join(CSRC, src)]
+                for obj, (src, defines) in zip(objs, OBJECTS)]
+        workers = int(os.environ.get("MAX_JOBS", 0)) or min(8, os.cpu_count() or 1)
+        with ThreadPoolExecutor(workers) as pool:
+            list(pool.map(run, jobs))
+        run([hipcc_path(), *flags, "-shared", "-o", tmp, *objs, "-lpthread"])
     os.replace(tmp, LIB_PATH)
     return LIB_PATH
 

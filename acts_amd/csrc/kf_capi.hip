@@ -14,7 +14,7 @@
 
 #include "kf_field_host.hpp"
 #include "kf_reference.hpp"
-#include "kf_reverse.hpp"
+#include "kf_forward.hpp"
 #include "kf_states.hpp"
 
 using namespace kf;
@@ -36,10 +36,6 @@ int fail(int code, const std::string& msg) {
                   std::string(#call) + ": " + hipGetErrorString(e_));         \
   } while (0)
 
-constexpr int kBlock = 64;
-// geometry kept in LDS by the forward kernel (224 B per surface)
-constexpr int kLdsSurfaces = 96;
-constexpr int kLdsSlabs = 32;
 // the track queue counts in int32 and may overshoot n by one per lane
 constexpr int64_t kMaxBatch = (int64_t{1} << 31) - (int64_t{1} << 24);
 
@@ -52,125 +48,6 @@ constexpr int64_t kMaxBatch = (int64_t{1} << 31) - (int64_t{1} << 24);
 constexpr size_t kStaticWorkspaceBytes = size_t{256} << 20;
 static __device__ __align__(256) unsigned char scratch[kStaticWorkspaceBytes];
 constexpr int kMaxDevices = 64;
-
-#ifndef KF_FORWARD_WAVES_PER_EU
-#define KF_FORWARD_WAVES_PER_EU 1
-#endif
-
-// Forward filter, persistent: each wavefront keeps its 64 lanes busy with
-// tracks taken from a global queue (`next`), in the order `order` when given
-// (longest surface sequence first, so that long tracks do not start last).
-// Per outer iteration: idle lanes
-// take new tracks; stepping lanes step until no lane steps any more, or at
-// least `waitFrac`/64 of the busy lanes wait at a surface, or `maxInner`
-// steps have been taken; then the waiting lanes run the surface update
-// together, and finished lanes write their summary and go idle.  With Rev
-// the kernel runs the reverse filter of the tracks that take one.  The
-// navigator is a template parameter (Layers: the layer navigator): its
-// option becomes a constant, so the direct navigator's instantiations carry
-// none of the layer navigator's code (a run-time choice cost the direct
-// fit's forward kernel 4 %).
-template <bool Mixed, bool GeoInLds, bool Sympy = false, bool Rev = false, bool Layers = false>
-__global__ __launch_bounds__(kBlock, KF_FORWARD_WAVES_PER_EU) void fitForwardKernel(
-    FwdArgs args, int32_t* __restrict__ next, int32_t maxInner, int32_t waitFrac,
-    int32_t quarantine, const int32_t* __restrict__ order) {
-  FwdArgs a = args;
-  a.o.navigator = Layers ? ACTS_KF_NAVIGATOR_LAYERS : ACTS_KF_NAVIGATOR_DIRECT;
-  const int lane = static_cast<int>(threadIdx.x) & 63;
-  // each lane's last field-map cell (cell-major maps): the first lookup of
-  // an RK step is nearly always in the cell of the previous step's last one
-  __shared__ double sCell[Mixed ? 1 : kCellValues * kCellCacheStride];
-  __shared__ float sCellF[Mixed ? kCellValues * kCellCacheStride : 1];
-  __shared__ int64_t sCellIdx[kCellCacheStride];
-  static_assert(kBlock == kCellCacheStride, "one cache column per lane of the workgroup");
-  a.F.cache = nullptr;
-  a.F.cacheF = nullptr;
-  a.F.cacheIdx = nullptr;
-  if (Mixed ? a.F.cellsF != nullptr : a.F.cells != nullptr) {
-    sCellIdx[lane] = -1;
-    if constexpr (Mixed)
-      a.F.cacheF = sCellF + lane;
-    else
-      a.F.cache = sCell + lane;
-    a.F.cacheIdx = sCellIdx + lane;
-  }
-  const uint64_t lanesBelow = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  const int64_t n = a.in.n;
-  // Surfaces and material slabs are read at every step: with GeoInLds (the
-  // geometry fits, as it does for the benchmark detectors) the workgroup
-  // keeps a copy in LDS.  The choice is a template parameter so that every
-  // geometry access compiles to an LDS read: a pointer that may point to
-  // either memory needs flat loads, which wait for all outstanding global
-  // loads and stores of the wavefront before their data can be used.
-  __shared__ DevSurface sGeo[GeoInLds ? kLdsSurfaces : 1];
-  __shared__ DevSlab sSlabs[GeoInLds ? kLdsSlabs : 1];
-  if constexpr (GeoInLds) {
-    const double* src = reinterpret_cast<const double*>(a.geo);
-    double* dst = reinterpret_cast<double*>(sGeo);
-    const int nd = a.nSurfaces * static_cast<int>(sizeof(DevSurface) / sizeof(double));
-    for (int i = static_cast<int>(threadIdx.x); i < nd; i += blockDim.x) dst[i] = src[i];
-    const int32_t* ss = reinterpret_cast<const int32_t*>(a.slabs);
-    int32_t* sd_ = reinterpret_cast<int32_t*>(sSlabs);
-    const int ns = a.nSlabs * static_cast<int>(sizeof(DevSlab) / sizeof(int32_t));
-    for (int i = static_cast<int>(threadIdx.x); i < ns; i += blockDim.x) sd_[i] = ss[i];
-    __syncthreads();
-  }
-  const DevSurface* geo = GeoInLds ? sGeo : a.geo;
-  const DevSlab* slabs = GeoInLds ? sSlabs : a.slabs;
-  Lane L;
-  int phase = kPhaseIdle;
-  while (true) {
-    // a wavefront holding a track that has run longer than `quarantine`
-    // steps takes no new tracks until it ends, so that the long track is not
-    // slowed down by the surface updates of fresh ones
-    const bool hold = quarantine > 0 &&
-                      __ballot(phase == kPhaseStepping && L.iter > static_cast<uint32_t>(quarantine)) != 0;
-    const uint64_t idle = hold ? 0ull : __ballot(phase == kPhaseIdle);
-    if (idle) {
-      const int cnt = __popcll(idle);
-      const int leader = __ffsll(static_cast<long long>(idle)) - 1;
-      int base = 0;
-      if (lane == leader) base = atomicAdd(next, cnt);
-      base = __shfl(base, leader);
-      if (phase == kPhaseIdle) {
-        const int64_t q = static_cast<int64_t>(base) + __popcll(idle & lanesBelow);
-        if (q >= n)
-          phase = kPhaseRetired;
-        else if constexpr (Rev)
-          phase = laneInitReverse<Mixed, Sympy>(L, q, order ? order[q] : q, a, geo);
-        else
-          phase = laneInit<Mixed, Sympy>(L, q, order ? order[q] : q, a, geo);
-      }
-    }
-    if (phase == kPhaseFinished) {
-      laneFinish<Rev>(L, a);
-      phase = kPhaseIdle;
-    }
-    const uint64_t busy = __ballot(phase != kPhaseRetired);
-    if (!busy) break;
-    for (int it = 0; it < maxInner; ++it) {
-      if (phase == kPhaseStepping) phase = laneStep<Mixed, Sympy, Rev>(L, a, geo);
-      const int nStep = __popcll(__ballot(phase == kPhaseStepping));
-      const int nWait = __popcll(__ballot(phase == kPhaseSurface || phase == kPhaseFinished));
-      if (nStep == 0 || 64 * nWait >= waitFrac * (nStep + nWait)) break;
-    }
-    // a lane that reached a surface while stepping without the transport
-    // goes back to its checkpoint and repeats the steps with it; a track
-    // that did so once (e.g. a looper that crosses a surface every turn)
-    // keeps the transport from then on
-    if (phase == kPhaseSurface && L.noTransport) {
-      L = a.ckpt[static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x];
-      L.replaying = true;
-      L.noSkip = true;
-      phase = kPhaseStepping;
-    }
-    if (phase == kPhaseSurface) phase = laneFilter<Mixed, Sympy, Rev>(L, a, geo, slabs);
-    if (phase == kPhaseFinished) {
-      laneFinish<Rev>(L, a);
-      phase = kPhaseIdle;
-    }
-  }
-}
 
 // Track-state table: one thread per row
 template <bool Sub>
@@ -204,12 +81,15 @@ __global__ __launch_bounds__(kBlock) void referenceKernel(DevOut out, DevScratch
                                                           int32_t strategy, int64_t n,
                                                           const int64_t* __restrict__ seqOff,
                                                           const int32_t* __restrict__ perm) {
+  __shared__ CellStore<Mixed> cells;
+  const CellCache cache = cellCache(cells, F);
   const int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   // failed fits, and reverse filters that reached the surface themselves
   if (q >= n || sc.track[q] != 0 || sc.track[2 * sc.stride + q] == kReferenceSet) return;
   const int64_t t = perm ? perm[q] : q;
   double p[6], C[36];
-  const int st = extrapolateTrack<Mixed, Sympy>(q, sc, sc.ref, geo, F, o, L, strategy, p, C);
+  const int st =
+      extrapolateTrack<Mixed, Sympy>(q, sc, sc.ref, geo, F, cache, o, L, strategy, p, C);
   if (st) {
     for (int64_t slot = seqOff[t]; slot < seqOff[t + 1]; ++slot) clearSlot(out, slot);
     if (out.status) out.status[t] = st;
@@ -687,45 +567,25 @@ int uploadFieldMap(acts_kf_ctx* c, const std::vector<double>& padded) {
   return r;
 }
 
-using ForwardFn = void (*)(FwdArgs, int32_t*, int32_t, int32_t, int32_t, const int32_t*);
-
 bool geometryFitsLds(const acts_kf_ctx* c) {
   return c->nSurfaces <= kLdsSurfaces && c->nSlabs <= kLdsSlabs;
 }
 
-template <bool Rev>
-ForwardFn forwardKernelOf(bool mixed, bool geoInLds, bool sympy, bool layers) {
-  if (layers) {
-    if (sympy && mixed)
-      return geoInLds ? fitForwardKernel<true, true, true, Rev, true>
-                      : fitForwardKernel<true, false, true, Rev, true>;
-    if (sympy)
-      return geoInLds ? fitForwardKernel<false, true, true, Rev, true>
-                      : fitForwardKernel<false, false, true, Rev, true>;
-    if (mixed)
-      return geoInLds ? fitForwardKernel<true, true, false, Rev, true>
-                      : fitForwardKernel<true, false, false, Rev, true>;
-    return geoInLds ? fitForwardKernel<false, true, false, Rev, true>
-                    : fitForwardKernel<false, false, false, Rev, true>;
-  }
-  if (sympy && mixed)
-    return geoInLds ? fitForwardKernel<true, true, true, Rev>
-                    : fitForwardKernel<true, false, true, Rev>;
-  if (sympy)
-    return geoInLds ? fitForwardKernel<false, true, true, Rev>
-                    : fitForwardKernel<false, false, true, Rev>;
-  if (mixed)
-    return geoInLds ? fitForwardKernel<true, true, false, Rev>
-                    : fitForwardKernel<true, false, false, Rev>;
-  return geoInLds ? fitForwardKernel<false, true, false, Rev>
-                  : fitForwardKernel<false, false, false, Rev>;
-}
 // the forward filter, or with `rev` the reverse filter, of a context
 ForwardFn forwardKernel(const acts_kf_ctx* c, bool rev = false) {
   const bool lds = geometryFitsLds(c);
   const bool layers = c->opts.navigator != ACTS_KF_NAVIGATOR_DIRECT;
-  return rev ? forwardKernelOf<true>(c->mixed, lds, c->sympy, layers)
-             : forwardKernelOf<false>(c->mixed, lds, c->sympy, layers);
+  if (c->mixed && c->sympy)
+    return layers ? forwardVariant<true, true, true>(lds, rev)
+                  : forwardVariant<true, true, false>(lds, rev);
+  if (c->mixed)
+    return layers ? forwardVariant<true, false, true>(lds, rev)
+                  : forwardVariant<true, false, false>(lds, rev);
+  if (c->sympy)
+    return layers ? forwardVariant<false, true, true>(lds, rev)
+                  : forwardVariant<false, true, false>(lds, rev);
+  return layers ? forwardVariant<false, false, true>(lds, rev)
+                : forwardVariant<false, false, false>(lds, rev);
 }
 
 }  // namespace
@@ -908,6 +768,9 @@ int acts_kf_create(const acts_kf_surface* surfaces, int32_t nSurfaces,
         c->field.minF[a] = static_cast<float>(c->field.min[a]);
         c->field.widthF[a] = static_cast<float>(c->field.width[a]);
         c->field.upperF[a] = static_cast<float>(c->field.upper[a]);
+        c->field.rwF[a] = 1.0f / c->field.widthF[a];
+        c->field.recipF = (a == 0 || c->field.recipF) && std::isnormal(c->field.widthF[a]) &&
+                          std::isnormal(c->field.rwF[a]);
       }
     }
     const int r = uploadFieldMap(c, padded);

@@ -243,7 +243,9 @@ struct DevField {
   // zero: [(ix * (nb1 + 1) + iy) * (nb2 + 1) + iz][3]
   const double* __restrict__ v;
   // the same map in float for the mixed-precision fit
-  float minF[3], widthF[3], upperF[3];
+  // (rwF = RN(1/widthF); recipF: those are normal numbers)
+  float minF[3], widthF[3], upperF[3], rwF[3];
+  int32_t recipF;
   int32_t pad3;
   const float* __restrict__ vf;
   // Cell-major copies of the map on the device (null: use the point arrays
@@ -255,13 +257,6 @@ struct DevField {
   // padding) instead of four point pairs in different cache lines.
   const double* __restrict__ cells;
   const float* __restrict__ cellsF;
-  // The lane's copy of the last cell record it read (the reference's cached
-  // FieldCell, InterpolatedBFieldMap.hpp:354-366), in LDS, value j at
-  // cache[j * kCellCacheStride] (cacheF for the FP32 map), and that cell's
-  // index at cacheIdx[0]; null (host code, kernels without it): no cache.
-  double* cache;
-  float* cacheF;
-  int64_t* cacheIdx;
 };
 // a / b rounded to nearest, from y = RN(1/b): q = a * y, then two
 // corrections q + (a - b q) y with fused multiply-adds.  The first makes q a
@@ -278,6 +273,28 @@ KF_HD double divRecip(double a, double b, double y) {
   q = fma(fma(-q, b, a), y, q);
   return fma(fma(-q, b, a), y, q);
 }
+
+// a / b from y = RN(1/b) in every case: the fix-up instruction gives the
+// results of the special operands (zeros with their sign, infinities, NaN).
+__device__ inline double divBy(double a, double b, double y) {
+  return __builtin_amdgcn_div_fixup(divRecip(a, b, y), b, a);
+}
+// normalized() with one division on the device: the three quotients by the
+// norm share its reciprocal.
+KF_HD V3 unit(const V3& a) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const double z = dot(a, a);
+  if (z > 0.0) {
+    const double n = sqrt(z);
+    const double y = 1.0 / n;
+    return mk(divBy(a.x, n, y), divBy(a.y, n, y), divBy(a.z, n, y));
+  }
+  return a;
+#else
+  return normalized(a);
+#endif
+}
+__device__ inline double divBy6(double a) { return divBy(a, 6.0, 1.0 / 6.0); }
 
 constexpr int kCellValues = 24;
 constexpr int kCellDoubles = 24;  // 192 B: two 128-byte cache lines

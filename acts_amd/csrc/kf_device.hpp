@@ -207,7 +207,7 @@ KF_HD V3 localToGlobal(const DevSurface& s, double l0, double l1) {
 KF_HD V3 cylinderNormal(const DevSurface& s, const V3& pos) {
   V3 p3 = toLocal(s, pos);
   p3.z = 0.;
-  return rotate(s.R, normalized(p3));
+  return rotate(s.R, unit(p3));
 }
 
 // The position part of the reference frame, columns x (fx), y (fy), z (fz).
@@ -220,7 +220,7 @@ KF_HD Frame referenceFrame(const DevSurface& s, const V3& pos) {
   if (s.type == ACTS_KF_SURFACE_CYLINDER) {
     f.fy = col(s.R, 2);
     f.fz = cylinderNormal(s, pos);
-    f.fx = normalized(cross(f.fy, f.fz));
+    f.fx = unit(cross(f.fy, f.fz));
   } else {
     f.fx = col(s.R, 0);
     f.fy = col(s.R, 1);
@@ -229,8 +229,7 @@ KF_HD Frame referenceFrame(const DevSurface& s, const V3& pos) {
   return f;
 }
 
-KF_HD double pathCorrection(const DevSurface& s, const V3& pos,
-                                        const V3& dir) {
+KF_HD double pathCorrection(const DevSurface& s, const V3& pos, const V3& dir) {
   if (s.type == ACTS_KF_SURFACE_CYLINDER) {
     const V3 n = cylinderNormal(s, pos);
     return fabs(1. / dot(n, dir));
@@ -241,8 +240,7 @@ KF_HD double pathCorrection(const DevSurface& s, const V3& pos,
 // Local-position columns of boundToFreeJacobian (rows 0..2, cols 0..1) and
 // local-position rows of freeToBoundJacobian (rows 0..1, cols 0..2).
 // Surface.cpp:249-290, DiscSurface.cpp:197-264.
-KF_HD void positionJacobians(const DevSurface& s, const V3& pos,
-                                         double b2f[6], double f2b[6]) {
+KF_HD void positionJacobians(const DevSurface& s, const V3& pos, double b2f[6], double f2b[6]) {
   if (s.type == ACTS_KF_SURFACE_DISC) {
     const V3 posLoc = toLocal(s, pos);
     const double lr = perp(posLoc);
@@ -308,6 +306,10 @@ struct Track {
   // derivative: (0..2) direction, (3) dt/ds, (4..6) k4
   double der[7];
   double pathAcc;
+  // What the steps need of the momentum, which changes only at a surface
+  // (setMomentum): dt/ds, and the denominator of d(time)/d(q/p) with its
+  // reciprocal; SympyStepper: also 1 / (q/p) and a third of it
+  double dtds, tden, trden, invQop, dirW;
   int nSteps, nTrials;
   // ConstrainedStep (ConstrainedStep.hpp:44-173)
   double cNav, cActor, cUser, cAcc;
@@ -370,26 +372,12 @@ KF_HD int gridField(const DevField& F, const V3& p, V3& out) {
   double c[4][3];
   if (F.cells) {
     const int64_t cell = (static_cast<int64_t>(lo[0]) * F.nb[1] + lo[1]) * F.nb[2] + lo[2];
-    double v[kCellValues];
-    if (F.cache && F.cacheIdx[0] == cell) {
-      // the lane's last cell: the same values without the gather
-#pragma unroll
-      for (int j = 0; j < kCellValues; ++j) v[j] = F.cache[j * kCellCacheStride];
-    } else {
-      const double* q = static_cast<const double*>(
-          __builtin_assume_aligned(F.cells + kCellDoubles * cell, 64));
-#pragma unroll
-      for (int j = 0; j < kCellValues; ++j) v[j] = q[j];
-      if (F.cache) {
-#pragma unroll
-        for (int j = 0; j < kCellValues; ++j) F.cache[j * kCellCacheStride] = v[j];
-        F.cacheIdx[0] = cell;
-      }
-    }
+    const double* q = static_cast<const double*>(
+        __builtin_assume_aligned(F.cells + kCellDoubles * cell, 64));
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int k = 0; k < 3; ++k) c[i][k] = (1 - f[2]) * v[6 * i + k] + f[2] * v[6 * i + 3 + k];
+      for (int k = 0; k < 3; ++k) c[i][k] = (1 - f[2]) * q[6 * i + k] + f[2] * q[6 * i + 3 + k];
   } else {
     const int64_t sy = F.nb[2] + 1;
     const int64_t sx = static_cast<int64_t>(F.nb[1] + 1) * (F.nb[2] + 1);
@@ -419,6 +407,107 @@ KF_HD int fieldAt(const DevField& F, const V3& p, V3& out) {
   return gridField(F, p, out);
 }
 
+// The field as a step looks it up.  A step is compiled once per kind of
+// field (withField), so that the three lookups of a trial are straight-line
+// code: tested per lookup, the field's kind, the reciprocals and every
+// axis's range cut them into short blocks, and the axes' chains of dependent
+// FP64 operations ran one after the other, with nothing beside them at one
+// wavefront per SIMD.  Measured with the shared reciprocals (divBy) and the
+// arguments read per phase (freshArgs): a fit of 500 000 field-map tracks
+// 12.8 -> 11.3 ms in FP64 and 11.3 -> 10.8 ms in mixed precision, of 5 000
+// tracks 7.7 -> 6.7 ms, 100 000 with SympyStepper and perigee 11.8 -> 9.6
+// ms; uniform field 6.6 -> 6.5 ms (100 000 tracks).  A lookup returns false
+// outside the map.
+struct UniformField {
+  V3 B;
+  __device__ inline bool operator()(const V3&, V3& out) const {
+    out = B;
+    return true;
+  }
+};
+
+// The lane's copy in LDS of the last cell record it read (the reference's
+// cached FieldCell, InterpolatedBFieldMap.hpp:354-366): value j at
+// v[j * kCellCacheStride] (vf for the FP32 map), the cell's index at idx[0];
+// null: no copy is kept.
+struct CellCache {
+  double* v;
+  float* vf;
+  int32_t* idx;
+};
+
+// A cell-major map whose axes allow the reciprocals (DevField::recip).
+struct CellField {
+  const DevField& F;
+  CellCache c;
+  __device__ inline bool operator()(const V3& p, V3& out) const {
+    out = mk(0.0, 0.0, 0.0);
+    const double x[3] = {p.x, p.y, p.z};
+    bool in = true;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) in = in & (x[a] >= F.min[a]) & !(x[a] >= F.upper[a]);
+    if (!in) return false;
+    // bin, lower edge and weight of each axis, as gridLocate
+    int lo[3];
+    double f[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const double u = divRecip(x[a] - F.min[a], F.width[a], F.rw[a]);
+      int bin = static_cast<int>(floor(u) + 1);
+      bin = bin < 1 ? 1 : (bin > F.nb[a] ? F.nb[a] : bin);
+      lo[a] = bin - 1;
+      const double ll = F.min[a] + static_cast<double>(bin - 1) * F.width[a];
+      f[a] = divRecip(x[a] - ll, F.den[a], F.rden[a]);
+    }
+    // kMaxCellBytes keeps the cell index within 32 bits
+    const int32_t cell = (lo[0] * F.nb[1] + lo[1]) * F.nb[2] + lo[2];
+    double v[kCellValues];
+    if (c.idx && c.idx[0] == cell) {
+#pragma unroll
+      for (int j = 0; j < kCellValues; ++j) v[j] = c.v[j * kCellCacheStride];
+    } else {
+      const double* q = static_cast<const double*>(
+          __builtin_assume_aligned(F.cells + static_cast<int64_t>(kCellDoubles) * cell, 64));
+#pragma unroll
+      for (int j = 0; j < kCellValues; ++j) v[j] = q[j];
+      if (c.idx) {
+#pragma unroll
+        for (int j = 0; j < kCellValues; ++j) c.v[j * kCellCacheStride] = v[j];
+        c.idx[0] = cell;
+      }
+    }
+    double e[4][3], d[2][3];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) e[i][k] = (1 - f[2]) * v[6 * i + k] + f[2] * v[6 * i + 3 + k];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) d[i][k] = (1 - f[1]) * e[2 * i][k] + f[1] * e[2 * i + 1][k];
+    out = mk((1 - f[0]) * d[0][0] + f[0] * d[1][0], (1 - f[0]) * d[0][1] + f[0] * d[1][1],
+             (1 - f[0]) * d[0][2] + f[0] * d[1][2]);
+    return true;
+  }
+};
+
+// Any other map: point arrays, axes that divide.
+struct AnyField {
+  const DevField& F;
+  __device__ inline bool operator()(const V3& p, V3& out) const {
+    out = mk(0.0, 0.0, 0.0);
+    return gridField(F, p, out) == 0;
+  }
+};
+
+// `step` with the accessor of the field's kind.
+template <typename Step>
+__device__ inline int withField(const DevField& F, const CellCache& c, Step&& step) {
+  if (F.kind == ACTS_KF_FIELD_CONSTANT) return step(UniformField{mk(F.B[0], F.B[1], F.B[2])});
+  if (F.cells && F.recip) return step(CellField{F, c});
+  return step(AnyField{F});
+}
+
 // EigenStepperDefaultExtension.hpp:40-58
 __device__ inline V3 kEval(double qop, const V3& dir, double h, const V3& kp,
                            const V3& B) {
@@ -445,7 +534,8 @@ struct RkStage {
 // is the propagation direction (+1 or -1): the step constraints are path
 // lengths along it, and the step is their value times the direction
 // (EigenStepper.ipp:270).
-__device__ inline int rkTrials(const Track& T, const DevField& F, const DevOpts& o, RkStage& S,
+template <typename Field>
+__device__ inline int rkTrials(const Track& T, const Field& field, const DevOpts& o, RkStage& S,
                                double propDir = 1.0) {
   S.pos = T.pos;
   S.dir = T.dir;
@@ -453,7 +543,7 @@ __device__ inline int rkTrials(const Track& T, const DevField& F, const DevOpts&
   const V3& pos = S.pos;
   const V3& dir = S.dir;
   const double qop = S.qop;
-  if (const int fs = fieldAt(F, pos, S.B1)) return fs;
+  if (!field(pos, S.B1)) return ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
   const V3 c1 = cross(dir, S.B1);
   S.k1 = mk(qop * c1.x, qop * c1.y, qop * c1.z);
   const V3& k1 = S.k1;
@@ -462,7 +552,9 @@ __device__ inline int rkTrials(const Track& T, const DevField& F, const DevOpts&
   S.initialH = h;
   double h2, half_h, err;
   int nTrials = 0;
-  while (true) {
+  int status = 0;
+  bool again;
+  do {
     ++nTrials;
     h2 = h * h;
     half_h = h * 0.5;
@@ -470,45 +562,62 @@ __device__ inline int rkTrials(const Track& T, const DevField& F, const DevOpts&
     const V3 p1 = mk((pos.x + half_h * dir.x) + h28 * k1.x,
                      (pos.y + half_h * dir.y) + h28 * k1.y,
                      (pos.z + half_h * dir.z) + h28 * k1.z);
-    if (const int fs = fieldAt(F, p1, S.B2)) return fs;
+    // a lookup outside the map ends the step below; what is computed in
+    // between is not used
+    bool inside = field(p1, S.B2);
     S.k2 = kEval(qop, dir, half_h, k1, S.B2);
     S.k3 = kEval(qop, dir, half_h, S.k2, S.B2);
     const double h22 = h2 * 0.5;
     const V3 p2 = mk((pos.x + h * dir.x) + h22 * S.k3.x,
                      (pos.y + h * dir.y) + h22 * S.k3.y,
                      (pos.z + h * dir.z) + h22 * S.k3.z);
-    if (const int fs = fieldAt(F, p2, S.B3)) return fs;
+    inside = field(p2, S.B3) & inside;
     S.k4 = kEval(qop, dir, h, S.k3, S.B3);
     const double e0 = ((k1.x - S.k2.x) - S.k3.x) + S.k4.x;
     const double e1 = ((k1.y - S.k2.y) - S.k3.y) + S.k4.y;
     const double e2 = ((k1.z - S.k2.z) - S.k3.z) + S.k4.z;
     err = h2 * ((fabs(e0) + fabs(e1)) + fabs(e2));
     err = fmax(1e-20, err);
-    if (err <= 4.0 * o.stepTolerance) break;
-    h *= stepScaling(o.stepTolerance, err);
-    if (fabs(h) < fabs(o.stepSizeCutOff)) return ACTS_KF_STATUS_STEP_SIZE_STALLED;
-    if (static_cast<uint32_t>(nTrials) > o.maxTrials)
-      return ACTS_KF_STATUS_STEP_ADJUSTMENT_FAILED;
-  }
+    again = inside && !(err <= 4.0 * o.stepTolerance);
+    if (again) {
+      h *= stepScaling(o.stepTolerance, err);
+      if (fabs(h) < fabs(o.stepSizeCutOff))
+        status = ACTS_KF_STATUS_STEP_SIZE_STALLED;
+      else if (static_cast<uint32_t>(nTrials) > o.maxTrials)
+        status = ACTS_KF_STATUS_STEP_ADJUSTMENT_FAILED;
+      again = status == 0;
+    }
+    if (!inside) status = ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
+  } while (again);
   S.h = h;
   S.h2 = h2;
   S.half_h = half_h;
   S.err = err;
   S.nTrials = nTrials;
-  return 0;
+  return status;
 }
 
-// propagateTime (EigenStepperDefaultExtension.hpp:112-125); returns dt/ds
-// and the momentum p used by the transport matrix.
-__device__ inline double rkTime(Track& T, const DevOpts& o, const RkStage& S, double& p) {
-  const float m = o.mass;
+// The momentum's part of propagateTime (EigenStepperDefaultExtension.hpp:
+// 112-125) and of d(time)/d(q/p): they depend on q/p alone, so they are
+// computed when it changes (at the start and after a surface's update), not
+// at every step.  With Sympy as SympyStepper.cpp has them.  tden times its
+// reciprocal gives the quotients the division by tden would (divBy).
+template <bool Sympy = false>
+__device__ inline void setMomentum(Track& T, const DevOpts& o) {
   // ParticleHypothesis::extractMomentum: float(copysign(|q|, q/p)) / (q/p)
-  p = copysign(static_cast<double>(o.absQ), S.qop) / S.qop;
-  const double mp = m / p;
-  const double dtds = sqrt(1 + mp * mp);
-  T.time += S.h * dtds;
-  T.der[3] = dtds;
-  return dtds;
+  const double p = copysign(static_cast<double>(o.absQ), T.qop) / T.qop;
+  const float m = o.mass;
+  if constexpr (Sympy) {
+    const double md = m;
+    T.dtds = sqrt(1 + (md * md) / (p * p));
+    T.invQop = 1 / T.qop;
+    T.dirW = T.invQop / 3;
+  } else {
+    const double mp = m / p;
+    T.dtds = sqrt(1 + mp * mp);
+  }
+  T.tden = p * p * T.qop * T.dtds;
+  T.trden = 1.0 / T.tden;
 }
 
 // d(k_i)/dT of the four stages, column j (j = 0..2) only.
@@ -567,7 +676,7 @@ __device__ inline void dkdL(const RkStage& S, V3& d1, V3& d2, V3& d3, V3& d4) {
 __device__ inline void dFdGColumn(const RkStage& S, int j, const double* c1, const double* c2,
                                   const double* c3, const double* c4, double out[6]) {
   const double h = S.h;
-  const double h6 = h / 6.;
+  const double h6 = divBy6(h);
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     const double id = (i == j ? 1.0 : 0.0);
@@ -578,8 +687,8 @@ __device__ inline void dFdGColumn(const RkStage& S, int j, const double* c1, con
 __device__ inline void dFdGLambda(const RkStage& S, const V3& d1, const V3& d2, const V3& d3,
                                   const V3& d4, double out[6]) {
   const double h = S.h;
-  const double h6 = h / 6.;
-  const double hh6 = (h * h) / 6.;
+  const double h6 = divBy6(h);
+  const double hh6 = divBy6(h * h);
   out[0] = hh6 * ((d1.x + d2.x) + d3.x);
   out[1] = hh6 * ((d1.y + d2.y) + d3.y);
   out[2] = hh6 * ((d1.z + d2.z) + d3.z);
@@ -587,9 +696,9 @@ __device__ inline void dFdGLambda(const RkStage& S, const V3& d1, const V3& d2, 
   out[4] = h6 * ((d1.y + 2. * (d2.y + d3.y)) + d4.y);
   out[5] = h6 * ((d1.z + 2. * (d2.z + d3.z)) + d4.z);
 }
-__device__ inline double transportD37(const DevOpts& o, const RkStage& S, double p, double dtds) {
+__device__ inline double transportD37(const Track& T, const DevOpts& o, double h) {
   const float m = o.mass;
-  return S.h * m * m / (p * p * S.qop * dtds);
+  return divBy(h * m * m, T.tden, T.trden);
 }
 
 // EigenStepper.ipp:341-347: TR += D_TR * BR ; BR = D_BR * BR, entry (i, j)
@@ -610,8 +719,7 @@ __device__ inline void blockEntry(int i, int j, const double* dFrow, const doubl
 }
 
 // The transport-matrix update of one accepted step, in one lane.
-__device__ inline void rkTransport(Track& T, const DevOpts& o, const RkStage& S, double p,
-                                   double dtds) {
+__device__ inline void rkTransport(Track& T, const DevOpts& o, const RkStage& S) {
   double col[4][6];
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
@@ -637,24 +745,26 @@ __device__ inline void rkTransport(Track& T, const DevOpts& o, const RkStage& S,
       T.br[4 * i + j] = nbr;
     }
   }
-  T.tr37 = T.tr37 + transportD37(o, S, p, dtds);
+  T.tr37 = T.tr37 + transportD37(T, o, S.h);
 }
 
-// EigenStepper.ipp:355-385: position, direction, derivative, path,
-// statistics, accuracy.
+// EigenStepper.ipp:325,355-385: time, position, direction, derivative,
+// path, statistics, accuracy.
 __device__ inline void rkApply(Track& T, const DevOpts& o, const RkStage& S) {
   const V3& pos = S.pos;
   const V3& dir = S.dir;
   const double h = S.h;
-  const double h6 = h / 6.;
-  const double h26 = S.h2 / 6.;
+  const double h6 = divBy6(h);
+  const double h26 = divBy6(S.h2);
+  T.time += h * T.dtds;
+  T.der[3] = T.dtds;
   T.pos = mk(pos.x + (h * dir.x + h26 * ((S.k1.x + S.k2.x) + S.k3.x)),
              pos.y + (h * dir.y + h26 * ((S.k1.y + S.k2.y) + S.k3.y)),
              pos.z + (h * dir.z + h26 * ((S.k1.z + S.k2.z) + S.k3.z)));
   V3 nd = mk(dir.x + h6 * ((S.k1.x + 2. * (S.k2.x + S.k3.x)) + S.k4.x),
              dir.y + h6 * ((S.k1.y + 2. * (S.k2.y + S.k3.y)) + S.k4.y),
              dir.z + h6 * ((S.k1.z + 2. * (S.k2.z + S.k3.z)) + S.k4.z));
-  T.dir = normalized(nd);
+  T.dir = unit(nd);
   T.der[0] = T.dir.x;
   T.der[1] = T.dir.y;
   T.der[2] = T.dir.z;
@@ -675,13 +785,12 @@ __device__ inline void rkApply(Track& T, const DevOpts& o, const RkStage& S) {
 // (EigenStepperDefaultExtension.hpp:137-228), propagation direction +1.
 // Without `transport` the step leaves the transport blocks (tr, tr37, br)
 // alone: the trajectory and the step-size control do not depend on them.
-__device__ inline int rkStep(Track& T, const DevField& F, const DevOpts& o,
+template <typename Field>
+__device__ inline int rkStep(Track& T, const Field& field, const DevOpts& o,
                              double propDir = 1.0, bool transport = true) {
   RkStage S;
-  if (const int st = rkTrials(T, F, o, S, propDir)) return st;
-  double p;
-  const double dtds = rkTime(T, o, S, p);
-  if (transport) rkTransport(T, o, S, p, dtds);
+  if (const int st = rkTrials(T, field, o, S, propDir)) return st;
+  if (transport) rkTransport(T, o, S);
   rkApply(T, o, S);
   return 0;
 }
@@ -722,23 +831,25 @@ __device__ inline V3 scale3(double s, const V3& a) { return mk(s * a.x, s * a.y,
 // tolerance; then the new position, normalised direction and time, and
 // (with `transport`) M's phi, theta and q/p columns through the same
 // recursion (tangents of the stages) and the path derivatives.
-__device__ inline int rkStepSympy(Track& T, const DevField& F, const DevOpts& o,
+template <typename Field>
+__device__ inline int rkStepSympy(Track& T, const Field& field, const DevOpts& o,
                                   double propDir = 1.0, bool transport = true) {
   const V3 pos = T.pos;
   const V3 dir = T.dir;
   const double qop = T.qop;
-  const double pabs = copysign(static_cast<double>(o.absQ), qop) / qop;
   const double m = o.mass;
   V3 B1;
-  if (const int fs = fieldAt(F, pos, B1)) return fs;
+  if (!field(pos, B1)) return ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
   const double initialH = stepValue(T) * propDir;
   double h = initialH, err = 0, hThird = 0;
   int nTrials = 0;
   V3 bend1, bend2, bend3, kick1, dir2, dir3, dir4, dirEnd, kick4;
-  while (true) {
+  int status = 0;
+  bool again;
+  do {
     ++nTrials;
     const double halfHQop = h * qop / 2;
-    hThird = h / 3;
+    hThird = divBy(h, 3.0, 1.0 / 3.0);
     const double hQuarter = h / 4;
     bend1 = scale3(halfHQop, B1);
     kick1 = cross(dir, bend1);
@@ -746,30 +857,37 @@ __device__ inline int rkStepSympy(Track& T, const DevField& F, const DevOpts& o,
     const V3 dirHalfSum = add3(dir2, dir);
     const V3 pos2 = add3(pos, scale3(hQuarter, dirHalfSum));
     V3 B2;
-    if (const int fs = fieldAt(F, pos2, B2)) return fs;
+    bool inside = field(pos2, B2);
     bend2 = scale3(halfHQop, B2);
     dir3 = add3(dir, cross(dir2, bend2));
     dir4 = add3(dir, cross(dir3, bend2));
     dirEnd = sub3(scale3(2, dir4), dir);
     const V3 pos3 = add3(pos, scale3(h, dir4));
     V3 B3;
-    if (const int fs = fieldAt(F, pos3, B3)) return fs;
+    inside = field(pos3, B3) & inside;
     bend3 = scale3(halfHQop, B3);
     kick4 = cross(dirEnd, bend3);
     const V3 e = sub3(add3(dirHalfSum, kick4), add3(dir3, dir4));
     err = 2 * fabs(h) * ((fabs(e.x) + fabs(e.y)) + fabs(e.z));
     const bool ok = !(err > 4.0 * o.stepTolerance);
     err = fmax(1e-20, err);
-    if (ok) break;
-    h *= stepScaling(o.stepTolerance, err);
-    if (fabs(h) < fabs(o.stepSizeCutOff)) return ACTS_KF_STATUS_STEP_SIZE_STALLED;
-    if (static_cast<uint32_t>(nTrials) > o.maxTrials) return ACTS_KF_STATUS_STEP_ADJUSTMENT_FAILED;
-  }
+    again = inside && !ok;
+    if (again) {
+      h *= stepScaling(o.stepTolerance, err);
+      if (fabs(h) < fabs(o.stepSizeCutOff))
+        status = ACTS_KF_STATUS_STEP_SIZE_STALLED;
+      else if (static_cast<uint32_t>(nTrials) > o.maxTrials)
+        status = ACTS_KF_STATUS_STEP_ADJUSTMENT_FAILED;
+      again = status == 0;
+    }
+    if (!inside) status = ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
+  } while (again);
+  if (status) return status;
   const V3 newPos = add3(pos, scale3(hThird, add3(add3(dir2, dir3), dir4)));
   const V3 newDirX3 = add3(scale3(2, dir3), add3(add3(kick1, dirEnd), kick4));
   const double invNorm = 1 / sqrt(dot(newDirX3, newDirX3));
   const V3 newDir = scale3(invNorm, newDirX3);
-  const double dtds = sqrt(1 + (m * m) / (pabs * pabs));
+  const double dtds = T.dtds;
   if (transport) {
     // phi and theta columns
 #pragma unroll
@@ -786,15 +904,14 @@ __device__ inline int rkStepSympy(Track& T, const DevField& F, const DevOpts& o,
       T.tr[c] = T.tr[c] + hThird * dp.x;
       T.tr[3 + c] = T.tr[3 + c] + hThird * dp.y;
       T.tr[6 + c] = T.tr[6 + c] + hThird * dp.z;
-      T.br[c] = dd.x / 3;
-      T.br[3 + c] = dd.y / 3;
-      T.br[6 + c] = dd.z / 3;
+      T.br[c] = divBy(dd.x, 3.0, 1.0 / 3.0);
+      T.br[3 + c] = divBy(dd.y, 3.0, 1.0 / 3.0);
+      T.br[6 + c] = divBy(dd.z, 3.0, 1.0 / 3.0);
     }
     // q/p column: direction part scaled by q/p plus the stages' own q/p
     // dependence (M(7, 4) = 1 in vacuum)
     {
-      const double invQop = 1 / qop;
-      const double posW = hThird * invQop, dirW = invQop / 3;
+      const double posW = hThird * T.invQop, dirW = T.dirW;
       const V3 seed = scale3(qop, mk(T.br[2], T.br[5], T.br[8]));
       const V3 tKick1 = add3(scale3(1.0, kick1), cross(seed, bend1));
       const V3 tDir2 = add3(tKick1, seed);
@@ -810,7 +927,7 @@ __device__ inline int rkStepSympy(Track& T, const DevField& F, const DevOpts& o,
       T.br[2] = dirW * dd.x;
       T.br[5] = dirW * dd.y;
       T.br[8] = dirW * dd.z;
-      const double dtDqop = h * (m * m) / ((pabs * pabs) * qop * dtds);
+      const double dtDqop = divBy(h * (m * m), T.tden, T.trden);
       T.tr37 = T.tr37 + dtDqop * 1.0;
     }
     const double twoOverH = 2 / h;

@@ -902,13 +902,12 @@ __device__ inline void layerNextTarget(Nav& nv, const Track& T, const DevSurface
 
 // Propagator.ipp:49-79.  `on`: the surface the track has just reached
 // (-1 none), which the layer navigator leaves out when it resolves again.
-template <bool Rev = false, typename SeqFn>
+template <bool Rev, bool Layers, typename SeqFn>
 __device__ inline int getNextTarget(Nav& nv, Track& T, const DevSurface* geo,
                                     const DevOpts& o, SeqFn seqAt, const LayerCtx& lc,
                                     int on) {
-  const bool layers = o.navigator != ACTS_KF_NAVIGATOR_DIRECT;
   for (uint32_t i = 0; i < o.maxTargetSkipping; ++i) {
-    if (layers)
+    if constexpr (Layers)
       layerNextTarget<Rev>(nv, T, geo, lc, on);
     else
       nextTarget<Rev>(nv, T, geo, o, seqAt);
@@ -916,7 +915,7 @@ __device__ inline int getNextTarget(Nav& nv, Track& T, const DevSurface* geo,
     on = -1;
     if (nv.tSurf < 0) return 0;
     const int st =
-        updateSurfaceStatus<Rev>(T, geo[nv.tSurf], nv.tIdx, o.surfaceTolerance, layers);
+        updateSurfaceStatus<Rev>(T, geo[nv.tSurf], nv.tIdx, o.surfaceTolerance, Layers);
     if (st == kOnSurface) continue;
     if (st == kReachable) return 0;
   }
@@ -924,28 +923,53 @@ __device__ inline int getNextTarget(Nav& nv, Track& T, const DevSurface* geo,
   return ACTS_KF_STATUS_NEXT_TARGET_LIMIT;
 }
 
-// LoopProtection.hpp:19-67 (forward)
-template <bool Mixed = false>
-__device__ inline void loopProtection(const Track& T, const DevField& F,
-                                      const DevOpts& o, double& limit,
-                                      bool release) {
-  if (!o.loopProtection) return;
-  if (release) limit = DBL_MAX;
-  // a failed lookup leaves the loop protection off (LoopProtection.hpp)
+// The path limit of the loop protection (LoopProtection.hpp:19-67): half a
+// turn of the helix at the present position, infinite where there is none
+// (no field, a failed lookup, switched off).
+template <bool Mixed>
+__device__ inline double loopLimit(const Track& T, const DevField& F, const DevOpts& o) {
+  if (!o.loopProtection) return INFINITY;
   V3 B;
+  int st;
   if constexpr (Mixed) {
     F3 b;
-    if (fieldAtF(F, tof(T.pos), b)) return;
+    st = withFieldF(F, CellCache{nullptr, nullptr, nullptr},
+                    [&](const auto& field) -> int { return !field(tof(T.pos), b); });
     B = mk(b.x, b.y, b.z);
   } else {
-    if (fieldAt(F, T.pos, B)) return;
+    st = fieldAt(F, T.pos, B);
   }
+  if (st) return INFINITY;
   const double Bn = sqrt(dot(B, B));
-  if (Bn == 0) return;
+  if (Bn == 0) return INFINITY;
   const double p = copysign(static_cast<double>(o.absQ), T.qop) / T.qop;
   const double helixPath = 2 * kPi * p / Bn;
-  const double loopLimit = o.loopFraction * helixPath;
-  if (fabs(loopLimit) < fabs(limit)) limit = loopLimit;
+  return o.loopFraction * helixPath;
+}
+
+// A limit on the path length, if it is the tighter one.
+__device__ inline void limitPath(double& limit, double v) {
+  if (fabs(v) < fabs(limit)) limit = v;
+}
+
+// One step of the chosen stepper and precision.
+template <bool Mixed, bool Sympy>
+__device__ inline int stepTrack(Track& T, const DevField& F, const CellCache& cache,
+                                const DevOpts& o, double propDir, bool transport) {
+  auto step = [&](const auto& field) -> int {
+    if constexpr (Mixed && Sympy)
+      return rkStepSympyMixed(T, field, o, propDir, transport);
+    else if constexpr (Mixed)
+      return rkStepMixed(T, field, o, propDir, transport);
+    else if constexpr (Sympy)
+      return rkStepSympy(T, field, o, propDir, transport);
+    else
+      return rkStep(T, field, o, propDir, transport);
+  };
+  if constexpr (Mixed)
+    return withFieldF(F, cache, step);
+  else
+    return withField(F, cache, step);
 }
 
 // PathLimitReached::checkAbort (StandardAborters.hpp:41-61)

@@ -111,6 +111,20 @@ __device__ inline LayerCtx layerCtx(const FwdArgs& a, int64_t q) {
                   a.sc.stride, a.nSurfaces};
 }
 
+// The forward kernel's arguments, read again from the kernel-argument
+// segment: the empty asm makes the compiler forget what it has loaded from
+// there.  The ~300 scalar registers' worth of options, field description and
+// pointers do not fit the 100 there are; loaded once before the persistent
+// loop they were parked in lanes of vector registers, 1 672 v_readlane and
+// v_writelane in the FP64 kernel, ~160 of them executed per step.  Called at
+// the start of a phase, what the phase needs comes from the scalar cache.
+__device__ inline const FwdArgs& freshArgs() {
+  using Args = const __attribute__((address_space(4))) FwdArgs;
+  uint64_t p = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const FwdArgs*)(Args*)p;
+}
+
 // The reverse filter's actor target check (SurfaceReached::checkAbort on the
 // reference surface) and the end of a reverse pass: kf_reverse.hpp.
 template <bool Sympy>
@@ -156,7 +170,7 @@ __device__ inline int uniqueMeasurementSurfaces(const DevBatch& in, int64_t m0, 
 // EigenStepper::initialize (EigenStepper.ipp:37-70), DirectNavigator
 // initialisation and the pre-propagation act of the KalmanFitter actor.
 // Returns the lane's next phase.
-template <bool Mixed, bool Sympy = false>
+template <bool Mixed, bool Sympy, bool Layers>
 __device__ inline int laneInit(Lane& L, const int64_t q, const int64_t t, const FwdArgs& a,
                                const DevSurface* geo) {
   const DevBatch& in = a.in;
@@ -188,7 +202,7 @@ __device__ inline int laneInit(Lane& L, const int64_t q, const int64_t t, const 
   // surface indices come from the caller: reject the track if any is out of
   // range instead of reading outside the geometry table
   bool badIndex = false;
-  if (o.navigator == ACTS_KF_NAVIGATOR_DIRECT) {
+  if constexpr (!Layers) {
     for (int i = 0; i < seqLen; ++i) {
       const int sid = L.seq(i);
       badIndex = badIndex || sid < 0 || sid >= a.nSurfaces;
@@ -233,34 +247,37 @@ __device__ inline int laneInit(Lane& L, const int64_t q, const int64_t t, const 
     T.cActor = kNotSet;
     T.cUser = o.maxStepSize;
     T.cAcc = o.initialStepSize;
+    setMomentum<Sympy>(T, o);
   }
-  L.nv.seqPos = o.navigator == ACTS_KF_NAVIGATOR_DIRECT ? -1 : kNavUnresolved;
+  L.nv.seqPos = Layers ? kNavUnresolved : -1;
   L.nv.seqLen = seqLen;
   L.nv.navBreak = false;
   L.nv.tSurf = -1;
   L.nv.tIdx = 0;
-  if (o.navigator != ACTS_KF_NAVIGATOR_DIRECT) clearReached(layerCtx(a, q));
+  if constexpr (Layers) clearReached(layerCtx(a, q));
 
+  const double loop = loopLimit<Mixed>(T, a.F, o);
   L.propLimit = o.pathLimit;
-  loopProtection<Mixed>(T, a.F, o, L.propLimit, false);
-  L.kfLimit = DBL_MAX;
+  limitPath(L.propLimit, loop);
   // pre-propagation act (the start surface carries neither material nor a
   // measurement, so only the finalisation checks run)
-  loopProtection<Mixed>(T, a.F, o, L.kfLimit, true);
+  L.kfLimit = DBL_MAX;
+  limitPath(L.kfLimit, loop);
   L.finished = (L.nMeasStates == L.nUnique) || pathAbort(T, L.kfLimit, o.surfaceTolerance);
   if (L.finished || pathAbort(T, L.propLimit, o.surfaceTolerance)) return kPhaseFinished;
-  L.status = getNextTarget(L.nv, T, geo, o, L.seq, layerCtx(a, q), -1);
+  L.status = getNextTarget<false, Layers>(L.nv, T, geo, o, L.seq, layerCtx(a, q), -1);
   return L.status ? kPhaseFinished : kPhaseStepping;
 }
 
-template <bool Mixed, bool Sympy = false, bool Rev = false>
+template <bool Mixed, bool Sympy, bool Rev, bool Layers>
 __device__ inline int laneAfterStep(Lane& L, const FwdArgs& a, const DevSurface* geo);
 
 // One iteration of the propagation loop (Propagator.ipp:25-210): step, target
 // status, the actor's finalisation checks, aborters, next target.  Rev: the
 // reverse filter, propagating backwards.
-template <bool Mixed, bool Sympy = false, bool Rev = false>
-__device__ inline int laneStep(Lane& L, const FwdArgs& a, const DevSurface* geo) {
+template <bool Mixed, bool Sympy, bool Rev, bool Layers>
+__device__ inline int laneStep(Lane& L, const FwdArgs& a, const DevSurface* geo,
+                               const CellCache& cache) {
   const DevOpts& o = a.o;
   Track& T = L.T;
   if (L.iter >= o.maxSteps) {
@@ -275,20 +292,12 @@ __device__ inline int laneStep(Lane& L, const FwdArgs& a, const DevSurface* geo)
   }
   ++L.iter;
   const bool transport = !L.noTransport;
-  int sst;
-  if constexpr (Mixed && Sympy)
-    sst = rkStepSympyMixed(T, a.F, o, propDir, transport);
-  else if constexpr (Mixed)
-    sst = rkStepMixed(T, a.F, o, propDir, transport);
-  else if constexpr (Sympy)
-    sst = rkStepSympy(T, a.F, o, propDir, transport);
-  else
-    sst = rkStep(T, a.F, o, propDir, transport);
+  const int sst = stepTrack<Mixed, Sympy>(T, a.F, cache, o, propDir, transport);
   if (sst) {
     L.status = sst;
     return kPhaseFinished;
   }
-  return laneAfterStep<Mixed, Sympy, Rev>(L, a, geo);
+  return laneAfterStep<Mixed, Sympy, Rev, Layers>(L, a, geo);
 }
 
 // The actor's finalisation checks (KalmanFitter.hpp:395-420): all
@@ -305,7 +314,7 @@ __device__ inline bool actorFinished(Lane& L, const FwdArgs& a) {
 
 // The rest of the propagation-loop iteration after an accepted step: target
 // status, the actor's finalisation checks, aborters, next target.
-template <bool Mixed, bool Sympy, bool Rev>
+template <bool Mixed, bool Sympy, bool Rev, bool Layers>
 __device__ inline int laneAfterStep(Lane& L, const FwdArgs& a, const DevSurface* geo) {
   const DevOpts& o = a.o;
   Track& T = L.T;
@@ -313,20 +322,20 @@ __device__ inline int laneAfterStep(Lane& L, const FwdArgs& a, const DevSurface*
   T.cActor = kNotSet;
   if (L.nv.tSurf >= 0) {
     const int ps = updateSurfaceStatus<Rev>(T, geo[L.nv.tSurf], L.nv.tIdx, o.surfaceTolerance,
-                                            o.navigator != ACTS_KF_NAVIGATOR_DIRECT);
+                                            Layers);
     if (ps == kOnSurface && !L.nv.navBreak) L.reached = L.nv.tSurf;
     if (ps != kReachable) L.nv.tSurf = -1;
   }
   if (L.reached >= 0) return kPhaseSurface;
   // act without a current surface: only the finalisation checks
   if (!L.finished) {
-    if (L.kfLimit == DBL_MAX) loopProtection<Mixed>(T, a.F, o, L.kfLimit, true);
+    if (L.kfLimit == DBL_MAX) limitPath(L.kfLimit, loopLimit<Mixed>(T, a.F, o));
     L.finished = actorFinished<Rev, Sympy>(L, a);
   }
   if (L.finished || pathAbort(T, L.propLimit, o.surfaceTolerance)) return kPhaseFinished;
   if (L.nv.tSurf < 0) {
     T.cNav = kNotSet;
-    L.status = getNextTarget<Rev>(L.nv, T, geo, o, L.seq, layerCtx(a, L.q), -1);
+    L.status = getNextTarget<Rev, Layers>(L.nv, T, geo, o, L.seq, layerCtx(a, L.q), -1);
     if (L.status) return kPhaseFinished;
   }
   return kPhaseStepping;
@@ -340,7 +349,7 @@ __device__ inline int laneAfterStep(Lane& L, const FwdArgs& a, const DevSurface*
 // after the update, backwards before it; on the reverse filter's start
 // surface only post-update material counts, which backwards is none
 // (PointwiseMaterialInteraction.cpp:16-29).
-template <bool Mixed, bool Sympy = false, bool Rev = false>
+template <bool Mixed, bool Sympy, bool Rev, bool Layers>
 __device__ inline int laneFilter(Lane& L, const FwdArgs& a, const DevSurface* geo,
                                  const DevSlab* slabs) {
   const DevBatch& in = a.in;
@@ -353,7 +362,7 @@ __device__ inline int laneFilter(Lane& L, const FwdArgs& a, const DevSurface* ge
   L.lastSurfIter = L.iter;
   L.replaying = false;
   if (!L.finished) {
-    if (L.kfLimit == DBL_MAX) loopProtection<Mixed>(T, a.F, o, L.kfLimit, true);
+    if (L.kfLimit == DBL_MAX) limitPath(L.kfLimit, loopLimit<Mixed>(T, a.F, o));
     const DevSurface& s = geo[reached];
     // the measurement on this surface: the first one in input order; when
     // all of the track's measurement surfaces differ and the measurements
@@ -486,6 +495,7 @@ __device__ inline int laneFilter(Lane& L, const FwdArgs& a, const DevSurface* ge
           // takes the full material in either direction
           if (matHere && (!Rev || mi < 0))
             L.status = materialInteraction(T, s, slabs[s.mat], a.pc, o, Rev ? -1.0 : 1.0);
+          setMomentum<Sympy>(T, o);
         }
       }
     }
@@ -494,7 +504,7 @@ __device__ inline int laneFilter(Lane& L, const FwdArgs& a, const DevSurface* ge
   }
   if (L.finished || pathAbort(T, L.propLimit, o.surfaceTolerance)) return kPhaseFinished;
   T.cNav = kNotSet;
-  L.status = getNextTarget<Rev>(L.nv, T, geo, o, L.seq, layerCtx(a, q), reached);
+  L.status = getNextTarget<Rev, Layers>(L.nv, T, geo, o, L.seq, layerCtx(a, q), reached);
   return L.status ? kPhaseFinished : kPhaseStepping;
 }
 

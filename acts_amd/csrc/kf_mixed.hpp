@@ -30,74 +30,106 @@ __device__ inline F3 crossf(const F3& a, const F3& b) {
   return F3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
 }
 
-// Trilinear lookup in the FP32 map (same cell, corner order and collapse
-// order as gridField).
-__device__ inline int gridFieldF(const DevField& F, const F3& p, F3& out) {
-  const float x[3] = {p.x, p.y, p.z};
-  int lo[3];
-  float f[3];
+// Trilinear interpolation of one cell's 24 values, the same corner and
+// collapse order as gridField.
+__device__ inline F3 interpolateF(const float v[kCellValues], const float f[3]) {
+  float c[4][3], d[2][3];
 #pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    const float mn = F.minF[a], w = F.widthF[a];
-    if (!(x[a] >= mn) || x[a] >= F.upperF[a]) return ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
-    int bin = static_cast<int>(floorf((x[a] - mn) / w) + 1.f);
-    bin = bin < 1 ? 1 : (bin > F.nb[a] ? F.nb[a] : bin);
-    lo[a] = bin - 1;
-    const float ll = mn + static_cast<float>(bin - 1) * w;
-    f[a] = (x[a] - ll) / w;
-  }
-  float c[4][3];
-  if (F.cellsF) {
-    // the cell's record: one 128-byte line
-    const int64_t cell = (static_cast<int64_t>(lo[0]) * F.nb[1] + lo[1]) * F.nb[2] + lo[2];
-    float v[kCellValues];
-    if (F.cacheF && F.cacheIdx[0] == cell) {
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < kCellValues; ++j) v[j] = F.cacheF[j * kCellCacheStride];
-    } else {
-      const float* q = static_cast<const float*>(
-          __builtin_assume_aligned(F.cellsF + kCellFloats * cell, 128));
-#pragma unroll
-      for (int j = 0; j < kCellValues; ++j) v[j] = q[j];
-      if (F.cacheF) {
-#pragma unroll
-        for (int j = 0; j < kCellValues; ++j) F.cacheF[j * kCellCacheStride] = v[j];
-        F.cacheIdx[0] = cell;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int k = 0; k < 3; ++k)
-        c[i][k] = (1.f - f[2]) * v[6 * i + k] + f[2] * v[6 * i + 3 + k];
-  } else {
-    const int64_t sy = F.nb[2] + 1;
-    const int64_t sx = static_cast<int64_t>(F.nb[1] + 1) * (F.nb[2] + 1);
-    const float* base = F.vf + 3 * (lo[0] * sx + lo[1] * sy + lo[2]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float* q = base + 3 * (((i >> 1) & 1) * sx + (i & 1) * sy);
-#pragma unroll
-      for (int k = 0; k < 3; ++k) c[i][k] = (1.f - f[2]) * q[k] + f[2] * q[3 + k];
-    }
-  }
-  float d[2][3];
+    for (int k = 0; k < 3; ++k) c[i][k] = (1.f - f[2]) * v[6 * i + k] + f[2] * v[6 * i + 3 + k];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int k = 0; k < 3; ++k) d[i][k] = (1.f - f[1]) * c[2 * i][k] + f[1] * c[2 * i + 1][k];
-  out = mkf((1.f - f[0]) * d[0][0] + f[0] * d[1][0], (1.f - f[0]) * d[0][1] + f[0] * d[1][1],
-            (1.f - f[0]) * d[0][2] + f[0] * d[1][2]);
-  return 0;
+  return mkf((1.f - f[0]) * d[0][0] + f[0] * d[1][0], (1.f - f[0]) * d[0][1] + f[0] * d[1][1],
+             (1.f - f[0]) * d[0][2] + f[0] * d[1][2]);
 }
 
-__device__ inline int fieldAtF(const DevField& F, const F3& p, F3& out) {
-  if (F.kind == ACTS_KF_FIELD_CONSTANT) {
-    out = mkf(static_cast<float>(F.B[0]), static_cast<float>(F.B[1]),
-              static_cast<float>(F.B[2]));
-    return 0;
+// The field accessors of the FP32 step (see UniformField in kf_device.hpp).
+struct UniformFieldF {
+  F3 B;
+  __device__ inline bool operator()(const F3&, F3& out) const {
+    out = B;
+    return true;
   }
-  return gridFieldF(F, p, out);
+};
+
+// a / b in FP32 from y = RN(1/b), as divRecip.
+__device__ inline float divRecipF(float a, float b, float y) {
+  float q = a * y;
+  q = fmaf(fmaf(-q, b, a), y, q);
+  return fmaf(fmaf(-q, b, a), y, q);
+}
+
+// The FP32 copy of the map.  Fast: a cell-major copy and widths whose
+// reciprocals are normal numbers (DevField::recipF); otherwise point arrays
+// may be read and the axes divide.
+template <bool Fast>
+struct MapFieldF {
+  const DevField& F;
+  CellCache c;
+  __device__ inline bool operator()(const F3& p, F3& out) const {
+    out = mkf(0.f, 0.f, 0.f);
+    const float x[3] = {p.x, p.y, p.z};
+    bool in = true;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) in = in & (x[a] >= F.minF[a]) & !(x[a] >= F.upperF[a]);
+    if (!in) return false;
+    int lo[3];
+    float f[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const float mn = F.minF[a], w = F.widthF[a];
+      const float u = Fast ? divRecipF(x[a] - mn, w, F.rwF[a]) : (x[a] - mn) / w;
+      int bin = static_cast<int>(floorf(u) + 1.f);
+      bin = bin < 1 ? 1 : (bin > F.nb[a] ? F.nb[a] : bin);
+      lo[a] = bin - 1;
+      const float ll = mn + static_cast<float>(bin - 1) * w;
+      f[a] = Fast ? divRecipF(x[a] - ll, w, F.rwF[a]) : (x[a] - ll) / w;
+    }
+    float v[kCellValues];
+    if (Fast || F.cellsF) {
+      // the cell's record, one 128-byte line; kMaxCellBytes keeps its index
+      // within 32 bits
+      const int32_t cell = (lo[0] * F.nb[1] + lo[1]) * F.nb[2] + lo[2];
+      if (c.idx && c.idx[0] == cell) {
+#pragma unroll
+        for (int j = 0; j < kCellValues; ++j) v[j] = c.vf[j * kCellCacheStride];
+      } else {
+        const float* q = static_cast<const float*>(
+            __builtin_assume_aligned(F.cellsF + static_cast<int64_t>(kCellFloats) * cell, 128));
+#pragma unroll
+        for (int j = 0; j < kCellValues; ++j) v[j] = q[j];
+        if (c.idx) {
+#pragma unroll
+          for (int j = 0; j < kCellValues; ++j) c.vf[j * kCellCacheStride] = v[j];
+          c.idx[0] = cell;
+        }
+      }
+    } else {
+      const int64_t sy = F.nb[2] + 1;
+      const int64_t sx = static_cast<int64_t>(F.nb[1] + 1) * (F.nb[2] + 1);
+      const float* base = F.vf + 3 * (lo[0] * sx + lo[1] * sy + lo[2]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float* q = base + 3 * (((i >> 1) & 1) * sx + (i & 1) * sy);
+#pragma unroll
+        for (int k = 0; k < 6; ++k) v[6 * i + k] = q[k];
+      }
+    }
+    out = interpolateF(v, f);
+    return true;
+  }
+};
+
+template <typename Step>
+__device__ inline int withFieldF(const DevField& F, const CellCache& c, Step&& step) {
+  if (F.kind == ACTS_KF_FIELD_CONSTANT)
+    return step(UniformFieldF{mkf(static_cast<float>(F.B[0]), static_cast<float>(F.B[1]),
+                                  static_cast<float>(F.B[2]))});
+  if (F.cellsF && F.recipF) return step(MapFieldF<true>{F, c});
+  return step(MapFieldF<false>{F, c});
 }
 
 __device__ inline float stepScalingF(float tol, float err) {
@@ -106,14 +138,15 @@ __device__ inline float stepScalingF(float tol, float err) {
   return fminf(fmaxf(x, 0.25f), 4.0f);
 }
 
-__device__ inline int rkStepMixed(Track& T, const DevField& F, const DevOpts& o,
+template <typename Field>
+__device__ inline int rkStepMixed(Track& T, const Field& field, const DevOpts& o,
                                   double propDir = 1.0, bool transport = true) {
   const F3 pos = tof(T.pos);
   const F3 dir = tof(T.dir);
   const float qop = static_cast<float>(T.qop);
   const float tol = static_cast<float>(o.stepTolerance);
   F3 B1;
-  if (const int fs = fieldAtF(F, pos, B1)) return fs;
+  if (!field(pos, B1)) return ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
   const F3 c1 = crossf(dir, B1);
   const F3 k1 = mkf(qop * c1.x, qop * c1.y, qop * c1.z);
 
@@ -125,14 +158,16 @@ __device__ inline int rkStepMixed(Track& T, const DevField& F, const DevOpts& o,
   float h2, half_h, err;
   F3 B2, B3, k2, k3, k4;
   int nTrials = 0;
-  while (true) {
+  int status = 0;
+  bool again;
+  do {
     ++nTrials;
     h2 = h * h;
     half_h = h * 0.5f;
     const float h28 = h2 * 0.125f;
     const F3 p1 = mkf((pos.x + half_h * dir.x) + h28 * k1.x, (pos.y + half_h * dir.y) + h28 * k1.y,
                       (pos.z + half_h * dir.z) + h28 * k1.z);
-    if (const int fs = fieldAtF(F, p1, B2)) return fs;
+    bool inside = field(p1, B2);
     F3 a = crossf(mkf(dir.x + half_h * k1.x, dir.y + half_h * k1.y, dir.z + half_h * k1.z), B2);
     k2 = mkf(qop * a.x, qop * a.y, qop * a.z);
     a = crossf(mkf(dir.x + half_h * k2.x, dir.y + half_h * k2.y, dir.z + half_h * k2.z), B2);
@@ -140,7 +175,7 @@ __device__ inline int rkStepMixed(Track& T, const DevField& F, const DevOpts& o,
     const float h22 = h2 * 0.5f;
     const F3 p2 = mkf((pos.x + h * dir.x) + h22 * k3.x, (pos.y + h * dir.y) + h22 * k3.y,
                       (pos.z + h * dir.z) + h22 * k3.z);
-    if (const int fs = fieldAtF(F, p2, B3)) return fs;
+    inside = field(p2, B3) & inside;
     a = crossf(mkf(dir.x + h * k3.x, dir.y + h * k3.y, dir.z + h * k3.z), B3);
     k4 = mkf(qop * a.x, qop * a.y, qop * a.z);
     const float e0 = ((k1.x - k2.x) - k3.x) + k4.x;
@@ -148,21 +183,25 @@ __device__ inline int rkStepMixed(Track& T, const DevField& F, const DevOpts& o,
     const float e2 = ((k1.z - k2.z) - k3.z) + k4.z;
     err = h2 * ((fabsf(e0) + fabsf(e1)) + fabsf(e2));
     err = fmaxf(1e-20f, err);
-    if (err <= 4.0f * tol) break;
-    h *= stepScalingF(tol, err);
-    hD = static_cast<double>(h);
-    if (fabs(hD) < fabs(o.stepSizeCutOff))
-      return ACTS_KF_STATUS_STEP_SIZE_STALLED;
-    if (static_cast<uint32_t>(nTrials) > o.maxTrials) return ACTS_KF_STATUS_STEP_ADJUSTMENT_FAILED;
-  }
+    again = inside && !(err <= 4.0f * tol);
+    if (again) {
+      h *= stepScalingF(tol, err);
+      hD = static_cast<double>(h);
+      if (fabs(hD) < fabs(o.stepSizeCutOff))
+        status = ACTS_KF_STATUS_STEP_SIZE_STALLED;
+      else if (static_cast<uint32_t>(nTrials) > o.maxTrials)
+        status = ACTS_KF_STATUS_STEP_ADJUSTMENT_FAILED;
+      again = status == 0;
+    }
+    if (!inside) status = ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
+  } while (again);
+  if (status) return status;
 
   // time and its derivatives in double (as rkTime): the time is not
   // measured, so its smoothed value is set by these jacobian entries through
   // the ill-conditioned RTS gain, which magnifies float rounding to ~1e-5
   const float m = o.mass;
-  const double pD = copysign(static_cast<double>(o.absQ), T.qop) / T.qop;
-  const double mpD = m / pD;
-  const double dtds = sqrt(1 + mpD * mpD);
+  const double dtds = T.dtds;
   T.time += hD * dtds;
   T.der[3] = dtds;
 
@@ -229,7 +268,7 @@ __device__ inline int rkStepMixed(Track& T, const DevField& F, const DevOpts& o,
   dG[3] = h6 * ((dk1dL.x + 2.f * (dk2dL.x + dk3dL.x)) + dk4dL.x);
   dG[7] = h6 * ((dk1dL.y + 2.f * (dk2dL.y + dk3dL.y)) + dk4dL.y);
   dG[11] = h6 * ((dk1dL.z + 2.f * (dk2dL.z + dk3dL.z)) + dk4dL.z);
-  const double D37 = hD * m * m / (pD * pD * T.qop * dtds);
+  const double D37 = divBy(hD * m * m, T.tden, T.trden);
 
   float br[12];
 #pragma unroll
@@ -292,7 +331,8 @@ __device__ inline int rkStepMixed(Track& T, const DevField& F, const DevOpts& o,
 // dir2 and dir3, and the q/p column's field terms dir3 - dir and dir4 - dir
 // are c2 and c3: the FP64 form's differences of O(1) vectors would leave
 // float noise of ~1e-7 in them.
-__device__ inline int rkStepSympyMixed(Track& T, const DevField& F, const DevOpts& o,
+template <typename Field>
+__device__ inline int rkStepSympyMixed(Track& T, const Field& field, const DevOpts& o,
                                        double propDir = 1.0, bool transport = true) {
   auto add = [](const F3& a, const F3& b) { return mkf(a.x + b.x, a.y + b.y, a.z + b.z); };
   auto sub = [](const F3& a, const F3& b) { return mkf(a.x - b.x, a.y - b.y, a.z - b.z); };
@@ -302,14 +342,16 @@ __device__ inline int rkStepSympyMixed(Track& T, const DevField& F, const DevOpt
   const float qop = static_cast<float>(T.qop);
   const float tol = static_cast<float>(o.stepTolerance);
   F3 B1;
-  if (const int fs = fieldAtF(F, pos, B1)) return fs;
+  if (!field(pos, B1)) return ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
   const double initialH = stepValue(T) * propDir;
   double hD = initialH;
   float h = static_cast<float>(initialH);
   float err, hThird;
   F3 bend1, bend2, bend3, kick1, c2, c3, kick4, dir2, dir3, dirEnd;
   int nTrials = 0;
-  while (true) {
+  int status = 0;
+  bool again;
+  do {
     ++nTrials;
     const float halfHQop = h * qop * 0.5f;
     hThird = h / 3.f;
@@ -319,7 +361,7 @@ __device__ inline int rkStepSympyMixed(Track& T, const DevField& F, const DevOpt
     dir2 = add(dir, kick1);
     const F3 pos2 = add(pos, scl(hQuarter, add(dir2, dir)));
     F3 B2;
-    if (const int fs = fieldAtF(F, pos2, B2)) return fs;
+    bool inside = field(pos2, B2);
     bend2 = scl(halfHQop, B2);
     c2 = crossf(dir2, bend2);
     dir3 = add(dir, c2);
@@ -328,22 +370,27 @@ __device__ inline int rkStepSympyMixed(Track& T, const DevField& F, const DevOpt
     dirEnd = sub(scl(2.f, dir4), dir);
     const F3 pos3 = add(pos, scl(h, dir4));
     F3 B3;
-    if (const int fs = fieldAtF(F, pos3, B3)) return fs;
+    inside = field(pos3, B3) & inside;
     bend3 = scl(halfHQop, B3);
     kick4 = crossf(dirEnd, bend3);
     const F3 e = add(sub(sub(kick1, c2), c3), kick4);
     err = 2.f * fabsf(h) * ((fabsf(e.x) + fabsf(e.y)) + fabsf(e.z));
     err = fmaxf(1e-20f, err);
-    if (err <= 4.0f * tol) break;
-    h *= stepScalingF(tol, err);
-    hD = static_cast<double>(h);
-    if (fabs(hD) < fabs(o.stepSizeCutOff)) return ACTS_KF_STATUS_STEP_SIZE_STALLED;
-    if (static_cast<uint32_t>(nTrials) > o.maxTrials) return ACTS_KF_STATUS_STEP_ADJUSTMENT_FAILED;
-  }
+    again = inside && !(err <= 4.0f * tol);
+    if (again) {
+      h *= stepScalingF(tol, err);
+      hD = static_cast<double>(h);
+      if (fabs(hD) < fabs(o.stepSizeCutOff))
+        status = ACTS_KF_STATUS_STEP_SIZE_STALLED;
+      else if (static_cast<uint32_t>(nTrials) > o.maxTrials)
+        status = ACTS_KF_STATUS_STEP_ADJUSTMENT_FAILED;
+      again = status == 0;
+    }
+    if (!inside) status = ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
+  } while (again);
+  if (status) return status;
   const float m = o.mass;
-  const double pD = copysign(static_cast<double>(o.absQ), T.qop) / T.qop;
-  const double mpD = m / pD;
-  const double dtds = sqrt(1 + mpD * mpD);
+  const double dtds = T.dtds;
   T.time += hD * dtds;
   if (transport) {
 #pragma unroll
@@ -384,7 +431,7 @@ __device__ inline int rkStepSympyMixed(Track& T, const DevField& F, const DevOpt
       T.br[2] = static_cast<double>(dirW * dd.x);
       T.br[5] = static_cast<double>(dirW * dd.y);
       T.br[8] = static_cast<double>(dirW * dd.z);
-      T.tr37 += hD * m * m / (pD * pD * T.qop * dtds);
+      T.tr37 += divBy(hD * m * m, T.tden, T.trden);
     }
   }
   // position: h dir in double, the bends (h/3)(kick1 + c2 + c3) in float;

@@ -211,6 +211,7 @@ __device__ inline void initializeFromBound(Track& T, const DevSurface& s, const 
   T.cActor = kNotSet;
   T.cUser = o.maxStepSize;
   T.cAcc = o.initialStepSize;
+  setMomentum<Sympy>(T, o);
 }
 
 // Propagator::propagate(start, target) to the line in direction `direction`
@@ -218,11 +219,12 @@ __device__ inline void initializeFromBound(Track& T, const DevSurface& s, const 
 // returns a status, T holds the state at the end.
 template <bool Mixed, bool Sympy = false>
 __device__ inline int propagateToLine(Track& T, const LineRef& L, const DevField& F,
-                                      const DevOpts& o, double direction) {
+                                      const CellCache& cache, const DevOpts& o,
+                                      double direction) {
   double limit = o.pathLimit;
   // setupLoopProtection: |limit| is what counts (PathLimitReached uses
   // |limit| - |path|), so the direction's sign does not enter
-  loopProtection<Mixed>(T, F, o, limit, false);
+  limitPath(limit, loopLimit<Mixed>(T, F, o));
   auto checkAbort = [&]() -> bool {
     // ForcedSurfaceReached::checkAbort: the intersection along the
     // propagation direction; near limit lowest, far limit max
@@ -238,15 +240,7 @@ __device__ inline int propagateToLine(Track& T, const LineRef& L, const DevField
   };
   if (checkAbort()) return 0;
   for (uint32_t steps = 0; steps < o.maxSteps; ++steps) {
-    int sst;
-    if constexpr (Mixed && Sympy)
-      sst = rkStepSympyMixed(T, F, o, direction);
-    else if constexpr (Mixed)
-      sst = rkStepMixed(T, F, o, direction);
-    else if constexpr (Sympy)
-      sst = rkStepSympy(T, F, o, direction);
-    else
-      sst = rkStep(T, F, o, direction);
+    const int sst = stepTrack<Mixed, Sympy>(T, F, cache, o, direction, true);
     if (sst) return sst;
     T.cNav = kNotSet;
     T.cActor = kNotSet;
@@ -261,8 +255,9 @@ __device__ inline int propagateToLine(Track& T, const LineRef& L, const DevField
 template <bool Mixed, bool Sympy = false>
 __device__ inline int extrapolateTrack(int64_t q, const DevScratch& sc, const double* ref,
                                        const DevSurface* geo, const DevField& F,
-                                       const DevOpts& o, const LineRef& L, int32_t strategy,
-                                       double params[6], double cov[36]) {
+                                       const CellCache& cache, const DevOpts& o,
+                                       const LineRef& L, int32_t strategy, double params[6],
+                                       double cov[36]) {
   const int first = sc.track[2 * sc.stride + q];
   const int last = sc.track[3 * sc.stride + q];
   if (first < 0) return ACTS_KF_STATUS_NO_COMPATIBLE_STATE;
@@ -304,7 +299,7 @@ __device__ inline int extrapolateTrack(int64_t q, const DevScratch& sc, const do
   const double direction = distance >= 0 ? 1.0 : -1.0;
   Track T;
   initializeFromBound<Sympy>(T, geo[si(sc, k, kISurf, q)], p, p + 6, o);
-  if (const int st = propagateToLine<Mixed, Sympy>(T, L, F, o, direction)) return st;
+  if (const int st = propagateToLine<Mixed, Sympy>(T, L, F, cache, o, direction)) return st;
   return lineBoundState<Sympy>(T, L, o.surfaceTolerance, params, cov);
 }
 

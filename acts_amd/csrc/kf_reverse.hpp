@@ -43,7 +43,7 @@ __device__ inline bool reverseWanted(const RevArgs& rv, const DevScratch& sc, in
 // first act is on the start surface, which is the navigator's current
 // surface (so the lane starts at the surface update).  Tracks that are not
 // filtered in reverse leave the lane idle.
-template <bool Mixed, bool Sympy = false>
+template <bool Mixed, bool Sympy, bool Layers>
 __device__ inline int laneInitReverse(Lane& L, const int64_t q, const int64_t t,
                                       const FwdArgs& a, const DevSurface* geo) {
   const DevScratch& sc = a.sc;
@@ -84,23 +84,22 @@ __device__ inline int laneInitReverse(Lane& L, const int64_t q, const int64_t t,
   initializeFromBound<Sympy>(T, geo[surf], p, p + 6, o);
   L.startSurf = surf;
   int found = -1;
-  if (o.navigator == ACTS_KF_NAVIGATOR_DIRECT)
+  if constexpr (!Layers)
     for (int i = 0; i < seqLen; ++i)
       if (found < 0 && L.seq(i) == surf) found = i;
   // the layer navigator resolves its lists without the start surface (the
   // volume's layer at the start position is the start object)
-  L.nv.seqPos = o.navigator == ACTS_KF_NAVIGATOR_DIRECT ? (found >= 0 ? found + 1 : seqLen)
-                                                       : kNavUnresolved;
+  L.nv.seqPos = Layers ? kNavUnresolved : (found >= 0 ? found + 1 : seqLen);
   L.nv.seqLen = seqLen;
   L.nv.navBreak = false;
   L.nv.tSurf = -1;
   L.nv.tIdx = 0;
-  if (o.navigator != ACTS_KF_NAVIGATOR_DIRECT) {
+  if constexpr (Layers) {
     clearReached(layerCtx(a, q));
     markReached(layerCtx(a, q), surf);
   }
   L.propLimit = o.pathLimit;
-  loopProtection<Mixed>(T, a.F, o, L.propLimit, false);
+  limitPath(L.propLimit, loopLimit<Mixed>(T, a.F, o));
   L.kfLimit = DBL_MAX;
   L.reached = surf;
   return kPhaseSurface;
