@@ -41,10 +41,10 @@ SPACE = {
     "sched_inner_steps": [8, 16, 32, 64, 128],
     "sched_wait_64ths": [16, 32, 48, 64],
     "length_sorted": [1, 0, 2, 3],
-    "sched_quarantine_steps": [0, 100, 200, 400],
+    "sched_quarantine_steps": [0, 100, 200, 400, -1],
     "sched_transport_skip_steps": [0, 64, 256],
 }
-DEFAULTS = {"sched_inner_steps": 64, "sched_wait_64ths": 64, "length_sorted": 1,
+DEFAULTS = {"sched_inner_steps": 16, "sched_wait_64ths": 64, "length_sorted": 1,
             "sched_quarantine_steps": 0, "sched_transport_skip_steps": 0}
 
 

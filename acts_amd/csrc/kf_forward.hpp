@@ -51,10 +51,13 @@ ForwardFn forwardVariant(bool geoInLds, bool rev);
 // tracks taken from a global queue (`next`), in the order `order` when given
 // (longest surface sequence first, so that long tracks do not start last).
 // Per outer iteration: idle lanes
-// take new tracks; stepping lanes step until no lane steps any more, or at
-// least `waitFrac`/64 of the busy lanes wait at a surface, or `maxInner`
-// steps have been taken; then the waiting lanes run the surface update
-// together, and finished lanes write their summary and go idle.  With Rev
+// take new tracks; stepping lanes step until no lane steps towards a surface
+// any more, or at least `waitFrac`/64 of the busy lanes wait at one, or
+// `maxInner` steps have been taken; then the waiting lanes run the surface
+// update together, and finished lanes write their summary and go idle.
+// Tracks past their last surface step on beside the others: waiting for
+// them, and stepping them with the transport, took 200 000 tracks with holes
+// and rejected outliers 7.4 instead of 3.4 ms here.  With Rev
 // the kernel runs the reverse filter of the tracks that take one.  The
 // navigator is a template parameter (Layers: the layer navigator): its
 // option becomes a constant, so the direct navigator's instantiations carry
@@ -96,10 +99,12 @@ __global__ __launch_bounds__(kBlock, 1) void fitForwardKernel(
   int phase = kPhaseIdle;
   while (true) {
     // a wavefront holding a track that has run longer than `quarantine`
-    // steps takes no new tracks until it ends, so that the long track is not
-    // slowed down by the surface updates of fresh ones
-    const bool hold = quarantine > 0 &&
-                      __ballot(phase == kPhaseStepping && L.iter > static_cast<uint32_t>(quarantine)) != 0;
+    // steps takes no new tracks until it ends, so that neither slows the
+    // other down: the long track waits for the surface updates of fresh ones,
+    // and they wait up to `maxInner` of its steps at every surface
+    const bool hold =
+        quarantine > 0 &&
+        __ballot(phase == kPhaseStepping && L.iter > static_cast<uint32_t>(quarantine)) != 0;
     const uint64_t idle = hold ? 0ull : __ballot(phase == kPhaseIdle);
     if (idle) {
       const int cnt = __popcll(idle);
@@ -126,9 +131,12 @@ __global__ __launch_bounds__(kBlock, 1) void fitForwardKernel(
     if (!busy) break;
     for (int it = 0; it < maxInner; ++it) {
       if (phase == kPhaseStepping) phase = laneStep<Mixed, Sympy, Rev, Layers>(L, freshArgs(), geo, cache);
-      const int nStep = __popcll(__ballot(phase == kPhaseStepping));
+      const bool stepping = phase == kPhaseStepping;
+      const int nStep = __popcll(__ballot(stepping && !pastLastSurface<Rev>(L)));
       const int nWait = __popcll(__ballot(phase == kPhaseSurface || phase == kPhaseFinished));
-      if (nStep == 0 || 64 * nWait >= waitFrac * (nStep + nWait)) break;
+      if (!__ballot(stepping) ||
+          (nWait > 0 && 64 * nWait >= waitFrac * (nStep + nWait)))
+        break;
     }
     // a lane that reached a surface while stepping without the transport
     // goes back to its checkpoint and repeats the steps with it; a track

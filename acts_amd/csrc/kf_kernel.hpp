@@ -269,6 +269,15 @@ __device__ inline int laneInit(Lane& L, const int64_t q, const int64_t t, const 
   return L.status ? kPhaseFinished : kPhaseStepping;
 }
 
+// A track whose navigation has ended (a rejected or unreached measurement
+// keeps its fit running to the path limit) reaches no surface any more: its
+// steps need no jacobian transport, and no other lane has to wait for it.
+// The reverse filter may still reach its target surface.
+template <bool Rev>
+__device__ inline bool pastLastSurface(const Lane& L) {
+  return !Rev && L.nv.navBreak && L.nv.tSurf < 0;
+}
+
 template <bool Mixed, bool Sympy, bool Rev, bool Layers>
 __device__ inline int laneAfterStep(Lane& L, const FwdArgs& a, const DevSurface* geo);
 
@@ -291,7 +300,7 @@ __device__ inline int laneStep(Lane& L, const FwdArgs& a, const DevSurface* geo,
     L.noTransport = true;
   }
   ++L.iter;
-  const bool transport = !L.noTransport;
+  const bool transport = !L.noTransport && !pastLastSurface<Rev>(L);
   const int sst = stepTrack<Mixed, Sympy>(T, a.F, cache, o, propDir, transport);
   if (sst) {
     L.status = sst;

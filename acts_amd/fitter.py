@@ -53,7 +53,7 @@ class KalmanFitterOptions:
     length_sorted: int = 1                  # queue order: 0 input, 1 length, 2 direction, 3 length+momentum
     sched_inner_steps: int = 0              # 0 = library default
     sched_wait_64ths: int = 0               # 0 = library default
-    sched_quarantine_steps: int = 0         # 0 = off
+    sched_quarantine_steps: int = 0         # 0 = library default, < 0 = off
     kernel_timing: bool = False             # events around the kernels
     use_graph: bool = False                 # replay fits as a captured hipGraph
     sched_transport_skip_steps: int = 0     # 0 = off

@@ -245,11 +245,12 @@ typedef struct acts_kf_options {
    *                   that neighbouring lanes bend alike); tracks with a
    *                   measurement near the +-pi seam of a cylinder first;
    * sched_inner_steps most RK steps the forward kernel takes before the
-   *                   lanes waiting at a surface are updated (0 = 64);
+   *                   lanes waiting at a surface are updated (0 = 16);
    * sched_wait_64ths  the surface update runs early once this many 64ths of
    *                   the busy lanes of a wavefront wait (0 = 64: all);
    * sched_quarantine_steps  a wavefront takes no new tracks while one of its
-   *                   tracks has run more than this many steps (0 = off).   */
+   *                   tracks has run more than this many steps (0 = 200,
+   *                   negative = off).                                      */
   int32_t length_sorted;
   int32_t sched_inner_steps;
   int32_t sched_wait_64ths;
