@@ -19,8 +19,8 @@ LIB_PATH = os.path.join(PKG_DIR, "libacts_kf.so")
 # (source, defines) of every object of the library; the forward kernel's
 # variants are compiled one by one
 OBJECTS = [("kf_capi.hip", []), ("generator.hip", [])] + [
-    ("kf_forward.hip", [f"-DKF_MIXED={m}", f"-DKF_SYMPY={s}", f"-DKF_LAYERS={n}"])
-    for m in (0, 1) for s in (0, 1) for n in (0, 1)]
+    ("kf_forward.hip", [f"-DKF_MIXED={m}", f"-DKF_SYMPY={s}", f"-DKF_LAYERS={n}", f"-DKF_MAP={f}"])
+    for m in (0, 1) for s in (0, 1) for n in (0, 1) for f in (0, 1)]
 HEADERS = ["kf_common.hpp", "kf_device.hpp", "kf_mixed.hpp", "kf_fit.hpp", "kf_kernel.hpp",
            "kf_reference.hpp", "kf_reverse.hpp", "kf_forward.hpp", "kf_states.hpp",
            "kf_field_host.hpp"]

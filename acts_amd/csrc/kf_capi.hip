@@ -74,7 +74,7 @@ __global__ __launch_bounds__(kBlock) void smoothKernel(DevBatch in, DevOut out,
 // surface, one lane per track (KalmanFitter.hpp:959-971).  A failure fails
 // the fit: the status becomes the extrapolation's error and the summary is
 // cleared, as for any failed fit.
-template <bool Mixed, bool Sympy = false>
+template <bool Mixed, bool Sympy, bool Map>
 __global__ __launch_bounds__(kBlock) void referenceKernel(DevOut out, DevScratch sc,
                                                           const DevSurface* __restrict__ geo,
                                                           DevField F, DevOpts o, LineRef L,
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(kBlock) void referenceKernel(DevOut out, DevScratch
   const int64_t t = perm ? perm[q] : q;
   double p[6], C[36];
   const int st =
-      extrapolateTrack<Mixed, Sympy>(q, sc, sc.ref, geo, F, cache, o, L, strategy, p, C);
+      extrapolateTrack<Mixed, Sympy, Map>(q, sc, sc.ref, geo, F, cache, o, L, strategy, p, C);
   if (st) {
     for (int64_t slot = seqOff[t]; slot < seqOff[t + 1]; ++slot) clearSlot(out, slot);
     if (out.status) out.status[t] = st;
@@ -580,21 +580,36 @@ bool geometryFitsLds(const acts_kf_ctx* c) {
   return c->nSurfaces <= kLdsSurfaces && c->nSlabs <= kLdsSlabs;
 }
 
+using ReferenceFn = void (*)(DevOut, DevScratch, const DevSurface*, DevField, DevOpts, LineRef,
+                             int32_t, int64_t, const int64_t*, const int32_t*);
+template <bool Mixed, bool Sympy>
+ReferenceFn referenceVariant(bool map) {
+  return map ? referenceKernel<Mixed, Sympy, true> : referenceKernel<Mixed, Sympy, false>;
+}
+ReferenceFn referenceKernelOf(const acts_kf_ctx* c) {
+  const bool map = c->field.kind != ACTS_KF_FIELD_CONSTANT;
+  if (c->mixed)
+    return c->sympy ? referenceVariant<true, true>(map) : referenceVariant<true, false>(map);
+  return c->sympy ? referenceVariant<false, true>(map) : referenceVariant<false, false>(map);
+}
+
 // the forward filter, or with `rev` the reverse filter, of a context
 ForwardFn forwardKernel(const acts_kf_ctx* c, bool rev = false) {
   const bool lds = geometryFitsLds(c);
   const bool layers = c->opts.navigator != ACTS_KF_NAVIGATOR_DIRECT;
-  if (c->mixed && c->sympy)
-    return layers ? forwardVariant<true, true, true>(lds, rev)
-                  : forwardVariant<true, true, false>(lds, rev);
-  if (c->mixed)
-    return layers ? forwardVariant<true, false, true>(lds, rev)
-                  : forwardVariant<true, false, false>(lds, rev);
-  if (c->sympy)
-    return layers ? forwardVariant<false, true, true>(lds, rev)
-                  : forwardVariant<false, true, false>(lds, rev);
-  return layers ? forwardVariant<false, false, true>(lds, rev)
-                : forwardVariant<false, false, false>(lds, rev);
+  const bool map = c->field.kind != ACTS_KF_FIELD_CONSTANT;
+  auto pick = [&](auto mixed, auto sympy) -> ForwardFn {
+    constexpr bool m = decltype(mixed)::value, s = decltype(sympy)::value;
+    if (layers)
+      return map ? forwardVariant<m, s, true, true>(lds, rev)
+                 : forwardVariant<m, s, true, false>(lds, rev);
+    return map ? forwardVariant<m, s, false, true>(lds, rev)
+               : forwardVariant<m, s, false, false>(lds, rev);
+  };
+  using No = std::false_type;
+  using Yes = std::true_type;
+  if (c->mixed) return c->sympy ? pick(Yes{}, Yes{}) : pick(Yes{}, No{});
+  return c->sympy ? pick(No{}, Yes{}) : pick(No{}, No{});
 }
 
 }  // namespace
@@ -1157,22 +1172,9 @@ static int launchFit(acts_kf_ctx* c, const acts_kf_batch_in* in,
                        c->innerSteps, c->waitFrac, 0, perm);
   }
   if (withRef) {
-    if (c->sympy && c->mixed)
-      hipLaunchKernelGGL((referenceKernel<true, true>), dim3(static_cast<unsigned>(blocks)),
-                         dim3(kBlock), 0, stream, d, sc, c->geo, c->field, c->extOpts,
-                         c->refLine, c->refStrategy, n, in->seq_offsets, perm);
-    else if (c->sympy)
-      hipLaunchKernelGGL((referenceKernel<false, true>), dim3(static_cast<unsigned>(blocks)),
-                         dim3(kBlock), 0, stream, d, sc, c->geo, c->field, c->extOpts,
-                         c->refLine, c->refStrategy, n, in->seq_offsets, perm);
-    else if (c->mixed)
-      hipLaunchKernelGGL(referenceKernel<true>, dim3(static_cast<unsigned>(blocks)), dim3(kBlock),
-                         0, stream, d, sc, c->geo, c->field, c->extOpts, c->refLine,
-                         c->refStrategy, n, in->seq_offsets, perm);
-    else
-      hipLaunchKernelGGL(referenceKernel<false>, dim3(static_cast<unsigned>(blocks)),
-                         dim3(kBlock), 0, stream, d, sc, c->geo, c->field, c->extOpts,
-                         c->refLine, c->refStrategy, n, in->seq_offsets, perm);
+    hipLaunchKernelGGL(referenceKernelOf(c), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0,
+                       stream, d, sc, c->geo, c->field, c->extOpts, c->refLine, c->refStrategy, n,
+                       in->seq_offsets, perm);
   }
   const hipError_t launchErr = hipGetLastError();
   if (graph) {

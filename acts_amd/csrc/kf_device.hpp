@@ -78,16 +78,25 @@ struct Isect {
   int size;
 };
 
-KF_HD Isect intersect(const DevSurface& s, const V3& pos,
-                                  const V3& dir, double tol) {
+// What the intersection with an unbounded surface needs of it.
+struct SurfaceLine {
+  V3 axis, t;  // third column of the rotation, translation
+  double b0;
+  int type;
+};
+KF_HD SurfaceLine surfaceLine(const DevSurface& s) {
+  return SurfaceLine{col(s.R, 2), mk(s.t[0], s.t[1], s.t[2]), s.b0, s.type};
+}
+
+KF_HD Isect intersect(const SurfaceLine& s, const V3& pos, const V3& dir, double tol) {
   Isect r;
   r.path[0] = r.path[1] = INFINITY;
   r.status[0] = r.status[1] = kUnreachable;
   if (s.type == ACTS_KF_SURFACE_CYLINDER) {
     // CylinderSurface.cpp:198-283, RealQuadraticEquation.hpp:57-66
     r.size = 2;
-    const V3 caxis = col(s.R, 2);
-    const V3 pc = mk(pos.x - s.t[0], pos.y - s.t[1], pos.z - s.t[2]);
+    const V3& caxis = s.axis;
+    const V3 pc = mk(pos.x - s.t.x, pos.y - s.t.y, pos.z - s.t.z);
     const V3 pcXcd = cross(pc, caxis);
     const V3 ldXcd = cross(dir, caxis);
     const double a = dot(ldXcd, ldXcd);
@@ -122,14 +131,16 @@ KF_HD Isect intersect(const DevSurface& s, const V3& pos,
   }
   // PlanarHelper.hpp:56-77
   r.size = 1;
-  const V3 n = col(s.R, 2);
+  const V3& n = s.axis;
   const double denom = dot(dir, n);
   if (denom == 0) return r;
-  const double path =
-      dot(n, mk(s.t[0] - pos.x, s.t[1] - pos.y, s.t[2] - pos.z)) / denom;
+  const double path = dot(n, mk(s.t.x - pos.x, s.t.y - pos.y, s.t.z - pos.z)) / denom;
   r.path[0] = path;
   r.status[0] = fabs(path) < fabs(tol) ? kOnSurface : kReachable;
   return r;
+}
+KF_HD Isect intersect(const DevSurface& s, const V3& pos, const V3& dir, double tol) {
+  return intersect(surfaceLine(s), pos, dir, tol);
 }
 
 // The bounds check of Surface::intersect with BoundaryTolerance::None at
@@ -407,12 +418,12 @@ KF_HD int fieldAt(const DevField& F, const V3& p, V3& out) {
   return gridField(F, p, out);
 }
 
-// The field as a step looks it up.  A step is compiled once per kind of
-// field (withField), so that the three lookups of a trial are straight-line
-// code: tested per lookup, the field's kind, the reciprocals and every
-// axis's range cut them into short blocks, and the axes' chains of dependent
-// FP64 operations ran one after the other, with nothing beside them at one
-// wavefront per SIMD.  Measured with the shared reciprocals (divBy) and the
+// The field as a step looks it up.  A step is compiled once for a uniform
+// field and once for a map, so that the three lookups of a trial are
+// straight-line code: tested per lookup, the field's kind, the reciprocals
+// and every axis's range cut them into short blocks, and the axes' chains of
+// dependent FP64 operations ran one after the other, with nothing beside
+// them at one wavefront per SIMD.  Measured with the shared reciprocals (divBy) and the
 // arguments read per phase (freshArgs): a fit of 500 000 field-map tracks
 // 12.8 -> 11.3 ms in FP64 and 11.3 -> 10.8 ms in mixed precision, of 5 000
 // tracks 7.7 -> 6.7 ms, 100 000 with SympyStepper and perigee 11.8 -> 9.6
@@ -436,12 +447,14 @@ struct CellCache {
   int32_t* idx;
 };
 
-// A cell-major map whose axes allow the reciprocals (DevField::recip).
-struct CellField {
+// A map: fast for a cell-major one whose axes allow the reciprocals
+// (DevField::recip), any other (point arrays, axes that divide) by gridField.
+struct MapField {
   const DevField& F;
   CellCache c;
   __device__ inline bool operator()(const V3& p, V3& out) const {
     out = mk(0.0, 0.0, 0.0);
+    if (!(F.cells && F.recip)) return gridField(F, p, out) == 0;
     const double x[3] = {p.x, p.y, p.z};
     bool in = true;
 #pragma unroll
@@ -490,23 +503,6 @@ struct CellField {
     return true;
   }
 };
-
-// Any other map: point arrays, axes that divide.
-struct AnyField {
-  const DevField& F;
-  __device__ inline bool operator()(const V3& p, V3& out) const {
-    out = mk(0.0, 0.0, 0.0);
-    return gridField(F, p, out) == 0;
-  }
-};
-
-// `step` with the accessor of the field's kind.
-template <typename Step>
-__device__ inline int withField(const DevField& F, const CellCache& c, Step&& step) {
-  if (F.kind == ACTS_KF_FIELD_CONSTANT) return step(UniformField{mk(F.B[0], F.B[1], F.B[2])});
-  if (F.cells && F.recip) return step(CellField{F, c});
-  return step(AnyField{F});
-}
 
 // EigenStepperDefaultExtension.hpp:40-58
 __device__ inline V3 kEval(double qop, const V3& dir, double h, const V3& kp,

@@ -759,11 +759,8 @@ __device__ inline V3 navDir(const Track& T) {
 // updateSingleSurfaceStatus (SteppingHelper.hpp:40-78): the direct
 // navigator's targets with BoundaryTolerance::Infinite, the layer
 // navigator's (bounded) with BoundaryTolerance::None.
-template <bool Rev = false>
-__device__ inline int updateSurfaceStatus(Track& T, const DevSurface& s, int idx,
-                                          double tol, bool bounded = false) {
-  const V3 d = navDir<Rev>(T);
-  const Isect x = bounded ? intersectBounded(s, T.pos, d, tol) : intersect(s, T.pos, d, tol);
+template <bool Rev>
+__device__ inline int updateSurfaceStatus(Track& T, const Isect& x, int idx) {
   const double path = idx ? x.path[1] : x.path[0];
   const int st = idx ? x.status[1] : x.status[0];
   if (st == kOnSurface) {
@@ -777,6 +774,14 @@ __device__ inline int updateSurfaceStatus(Track& T, const DevSurface& s, int idx
     return kReachable;
   }
   return kUnreachable;
+}
+
+// The intersection of the track's line with its target.
+template <bool Rev, bool Layers>
+__device__ inline Isect targetIntersection(const Track& T, const DevSurface& s, const DevOpts& o) {
+  const V3 d = navDir<Rev>(T);
+  if constexpr (Layers) return intersectBounded(s, T.pos, d, o.surfaceTolerance);
+  return intersect(s, T.pos, d, o.surfaceTolerance);
 }
 
 // nextSurface / endOfSurfaces (DirectNavigator.hpp:107-124): the sequence
@@ -915,7 +920,7 @@ __device__ inline int getNextTarget(Nav& nv, Track& T, const DevSurface* geo,
     on = -1;
     if (nv.tSurf < 0) return 0;
     const int st =
-        updateSurfaceStatus<Rev>(T, geo[nv.tSurf], nv.tIdx, o.surfaceTolerance, Layers);
+        updateSurfaceStatus<Rev>(T, targetIntersection<Rev, Layers>(T, geo[nv.tSurf], o), nv.tIdx);
     if (st == kOnSurface) continue;
     if (st == kReachable) return 0;
   }
@@ -933,8 +938,7 @@ __device__ inline double loopLimit(const Track& T, const DevField& F, const DevO
   int st;
   if constexpr (Mixed) {
     F3 b;
-    st = withFieldF(F, CellCache{nullptr, nullptr, nullptr},
-                    [&](const auto& field) -> int { return !field(tof(T.pos), b); });
+    st = fieldAtF(F, tof(T.pos), b);
     B = mk(b.x, b.y, b.z);
   } else {
     st = fieldAt(F, T.pos, B);
@@ -952,8 +956,9 @@ __device__ inline void limitPath(double& limit, double v) {
   if (fabs(v) < fabs(limit)) limit = v;
 }
 
-// One step of the chosen stepper and precision.
-template <bool Mixed, bool Sympy>
+// One step of the chosen stepper and precision in a uniform field, or (Map)
+// in a field map.
+template <bool Mixed, bool Sympy, bool Map>
 __device__ inline int stepTrack(Track& T, const DevField& F, const CellCache& cache,
                                 const DevOpts& o, double propDir, bool transport) {
   auto step = [&](const auto& field) -> int {
@@ -966,10 +971,15 @@ __device__ inline int stepTrack(Track& T, const DevField& F, const CellCache& ca
     else
       return rkStep(T, field, o, propDir, transport);
   };
-  if constexpr (Mixed)
-    return withFieldF(F, cache, step);
+  if constexpr (Map && Mixed)
+    return step(MapFieldF{F, cache});
+  else if constexpr (Map)
+    return step(MapField{F, cache});
+  else if constexpr (Mixed)
+    return step(UniformFieldF{mkf(static_cast<float>(F.B[0]), static_cast<float>(F.B[1]),
+                                  static_cast<float>(F.B[2]))});
   else
-    return withField(F, cache, step);
+    return step(UniformField{mk(F.B[0], F.B[1], F.B[2])});
 }
 
 // PathLimitReached::checkAbort (StandardAborters.hpp:41-61)

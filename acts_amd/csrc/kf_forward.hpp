@@ -2,7 +2,7 @@
 // Rev the reverse filter).
 //
 // Its instantiations are compiled apart (kf_forward.hip, one object per
-// precision, stepper and navigator), so that they build in parallel; the
+// precision, stepper, navigator and field), so that they build in parallel; the
 // host code reaches them through forwardVariant.
 #pragma once
 
@@ -42,9 +42,9 @@ __device__ inline CellCache cellCache(CellStore<Mixed>& s, const DevField& F) {
 
 using ForwardFn = void (*)(FwdArgs, int32_t*, int32_t, int32_t, int32_t, const int32_t*);
 
-// The kernel of a precision, stepper and navigator: geometry in LDS or in
-// global memory, forward or reverse filter.
-template <bool Mixed, bool Sympy, bool Layers>
+// The kernel of a precision, stepper, navigator and kind of field: geometry
+// in LDS or in global memory, forward or reverse filter.
+template <bool Mixed, bool Sympy, bool Layers, bool Map>
 ForwardFn forwardVariant(bool geoInLds, bool rev);
 
 // Forward filter, persistent: each wavefront keeps its 64 lanes busy with
@@ -62,8 +62,10 @@ ForwardFn forwardVariant(bool geoInLds, bool rev);
 // navigator is a template parameter (Layers: the layer navigator): its
 // option becomes a constant, so the direct navigator's instantiations carry
 // none of the layer navigator's code (a run-time choice cost the direct
-// fit's forward kernel 4 %).
-template <bool Mixed, bool GeoInLds, bool Sympy, bool Rev, bool Layers>
+// fit's forward kernel 4 %).  So is the kind of field (Map): with a step per
+// kind in one kernel, ~100 of the ~1 100 vector instructions of a step in a
+// uniform field were moves that brought the kinds' results together.
+template <bool Mixed, bool GeoInLds, bool Sympy, bool Rev, bool Layers, bool Map>
 __global__ __launch_bounds__(kBlock, 1) void fitForwardKernel(
     FwdArgs args, int32_t* __restrict__ next, int32_t maxInner, int32_t waitFrac,
     int32_t quarantine, const int32_t* __restrict__ order) {
@@ -129,8 +131,11 @@ __global__ __launch_bounds__(kBlock, 1) void fitForwardKernel(
     }
     const uint64_t busy = __ballot(phase != kPhaseRetired);
     if (!busy) break;
+    const FwdArgs& as = freshArgs();
+    const StepArgs sa = stepArgs<Mixed, Map>(as);
     for (int it = 0; it < maxInner; ++it) {
-      if (phase == kPhaseStepping) phase = laneStep<Mixed, Sympy, Rev, Layers>(L, freshArgs(), geo, cache);
+      if (phase == kPhaseStepping)
+        phase = laneStep<Mixed, Sympy, Rev, Layers, Map>(L, as, sa, geo, cache);
       const bool stepping = phase == kPhaseStepping;
       const int nStep = __popcll(__ballot(stepping && !pastLastSurface<Rev>(L)));
       const int nWait = __popcll(__ballot(phase == kPhaseSurface || phase == kPhaseFinished));

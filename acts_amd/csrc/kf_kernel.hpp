@@ -105,6 +105,46 @@ struct FwdArgs {
   RevArgs rv;
 };
 
+// The arguments a step uses, kept in scalar registers while a wavefront
+// steps (the empty asm makes their values ones that cannot be read again).
+// Left to the compiler each is read where it is used, 7 reads a step in a
+// uniform field and 35 in a map, and a wavefront that is alone on its SIMD
+// stands still for every one of them.
+struct StepArgs {
+  DevOpts o;
+  DevField F;
+  int32_t skipAfter;
+};
+template <bool Mixed, bool Map>
+__device__ inline StepArgs stepArgs(const FwdArgs& a) {
+  StepArgs s;
+  s.o = a.o;
+  s.F = a.F;
+  s.skipAfter = a.skipAfter;
+  asm volatile("" : "+s"(s.o.stepTolerance), "+s"(s.o.stepSizeCutOff),
+                    "+s"(s.o.surfaceTolerance), "+s"(s.o.maxTrials), "+s"(s.o.maxSteps),
+                    "+s"(s.o.mass), "+s"(s.skipAfter));
+  DevField& F = s.F;
+  if constexpr (!Map) {
+    asm volatile("" : "+s"(F.B[0]), "+s"(F.B[1]), "+s"(F.B[2]));
+  } else if constexpr (Mixed) {
+    asm volatile("" : "+s"(F.minF[0]), "+s"(F.minF[1]), "+s"(F.minF[2]), "+s"(F.upperF[0]),
+                      "+s"(F.upperF[1]), "+s"(F.upperF[2]), "+s"(F.widthF[0]),
+                      "+s"(F.widthF[1]), "+s"(F.widthF[2]), "+s"(F.rwF[0]), "+s"(F.rwF[1]),
+                      "+s"(F.rwF[2]));
+    asm volatile("" : "+s"(F.nb[0]), "+s"(F.nb[1]), "+s"(F.nb[2]), "+s"(F.cellsF),
+                      "+s"(F.recipF));
+  } else {
+    asm volatile("" : "+s"(F.min[0]), "+s"(F.min[1]), "+s"(F.min[2]), "+s"(F.upper[0]),
+                      "+s"(F.upper[1]), "+s"(F.upper[2]), "+s"(F.width[0]), "+s"(F.width[1]),
+                      "+s"(F.width[2]), "+s"(F.rw[0]), "+s"(F.rw[1]), "+s"(F.rw[2]));
+    asm volatile("" : "+s"(F.den[0]), "+s"(F.den[1]), "+s"(F.den[2]), "+s"(F.rden[0]),
+                      "+s"(F.rden[1]), "+s"(F.rden[2]), "+s"(F.nb[0]), "+s"(F.nb[1]),
+                      "+s"(F.nb[2]), "+s"(F.cells), "+s"(F.recip));
+  }
+  return s;
+}
+
 // The layer-navigator record of queue slot q.
 __device__ inline LayerCtx layerCtx(const FwdArgs& a, int64_t q) {
   return LayerCtx{a.sc.nav ? a.sc.nav + q : nullptr, a.sc.nav ? a.sc.navMask + q : nullptr,
@@ -279,42 +319,46 @@ __device__ inline bool pastLastSurface(const Lane& L) {
 }
 
 template <bool Mixed, bool Sympy, bool Rev, bool Layers>
-__device__ inline int laneAfterStep(Lane& L, const FwdArgs& a, const DevSurface* geo);
+__device__ inline int laneAfterStep(Lane& L, const FwdArgs& a, const DevOpts& o,
+                                    const DevSurface* geo, const SurfaceLine& target);
 
 // One iteration of the propagation loop (Propagator.ipp:25-210): step, target
 // status, the actor's finalisation checks, aborters, next target.  Rev: the
 // reverse filter, propagating backwards.
-template <bool Mixed, bool Sympy, bool Rev, bool Layers>
-__device__ inline int laneStep(Lane& L, const FwdArgs& a, const DevSurface* geo,
-                               const CellCache& cache) {
-  const DevOpts& o = a.o;
+template <bool Mixed, bool Sympy, bool Rev, bool Layers, bool Map>
+__device__ inline int laneStep(Lane& L, const FwdArgs& a, const StepArgs& s,
+                               const DevSurface* geo, const CellCache& cache) {
+  const DevOpts& o = s.o;
   Track& T = L.T;
+  // the target's geometry for the intersection after the step, read before
+  // it, so that the step's arithmetic covers the wait
+  const SurfaceLine target = surfaceLine(geo[L.nv.tSurf >= 0 ? L.nv.tSurf : 0]);
   if (L.iter >= o.maxSteps) {
     L.status = ACTS_KF_STATUS_STEP_COUNT_LIMIT;
     return kPhaseFinished;
   }
   constexpr double propDir = Rev ? -1.0 : 1.0;
-  if (!Rev && a.skipAfter > 0 && !L.noTransport && !L.replaying && !L.noSkip &&
-      L.iter - L.lastSurfIter >= static_cast<uint32_t>(a.skipAfter)) {
+  if (!Rev && s.skipAfter > 0 && !L.noTransport && !L.replaying && !L.noSkip &&
+      L.iter - L.lastSurfIter >= static_cast<uint32_t>(s.skipAfter)) {
     a.ckpt[static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x] = L;
     L.noTransport = true;
   }
   ++L.iter;
   const bool transport = !L.noTransport && !pastLastSurface<Rev>(L);
-  const int sst = stepTrack<Mixed, Sympy>(T, a.F, cache, o, propDir, transport);
+  const int sst = stepTrack<Mixed, Sympy, Map>(T, s.F, cache, o, propDir, transport);
   if (sst) {
     L.status = sst;
     return kPhaseFinished;
   }
-  return laneAfterStep<Mixed, Sympy, Rev, Layers>(L, a, geo);
+  return laneAfterStep<Mixed, Sympy, Rev, Layers>(L, a, o, geo, target);
 }
 
 // The actor's finalisation checks (KalmanFitter.hpp:395-420): all
 // measurements handled, the path limit, and for the reverse filter its
 // target (each check updates the actor step size, in this order).
 template <bool Rev, bool Sympy>
-__device__ inline bool actorFinished(Lane& L, const FwdArgs& a) {
-  bool fin = (L.nMeasStates == L.nUnique) || pathAbort(L.T, L.kfLimit, a.o.surfaceTolerance);
+__device__ inline bool actorFinished(Lane& L, const FwdArgs& a, const DevOpts& o) {
+  bool fin = (L.nMeasStates == L.nUnique) || pathAbort(L.T, L.kfLimit, o.surfaceTolerance);
   if constexpr (Rev) {
     if (a.rv.hasTarget) fin = reverseTargetReached<Sympy>(L, a) || fin;
   }
@@ -324,27 +368,31 @@ __device__ inline bool actorFinished(Lane& L, const FwdArgs& a) {
 // The rest of the propagation-loop iteration after an accepted step: target
 // status, the actor's finalisation checks, aborters, next target.
 template <bool Mixed, bool Sympy, bool Rev, bool Layers>
-__device__ inline int laneAfterStep(Lane& L, const FwdArgs& a, const DevSurface* geo) {
-  const DevOpts& o = a.o;
+__device__ inline int laneAfterStep(Lane& L, const FwdArgs& a, const DevOpts& o,
+                                    const DevSurface* geo, const SurfaceLine& target) {
   Track& T = L.T;
   T.cNav = kNotSet;
   T.cActor = kNotSet;
   if (L.nv.tSurf >= 0) {
-    const int ps = updateSurfaceStatus<Rev>(T, geo[L.nv.tSurf], L.nv.tIdx, o.surfaceTolerance,
-                                            Layers);
+    Isect x;
+    if constexpr (Layers)
+      x = targetIntersection<Rev, true>(T, geo[L.nv.tSurf], o);
+    else
+      x = intersect(target, T.pos, navDir<Rev>(T), o.surfaceTolerance);
+    const int ps = updateSurfaceStatus<Rev>(T, x, L.nv.tIdx);
     if (ps == kOnSurface && !L.nv.navBreak) L.reached = L.nv.tSurf;
     if (ps != kReachable) L.nv.tSurf = -1;
   }
   if (L.reached >= 0) return kPhaseSurface;
   // act without a current surface: only the finalisation checks
   if (!L.finished) {
-    if (L.kfLimit == DBL_MAX) limitPath(L.kfLimit, loopLimit<Mixed>(T, a.F, o));
-    L.finished = actorFinished<Rev, Sympy>(L, a);
+    if (L.kfLimit == DBL_MAX) limitPath(L.kfLimit, loopLimit<Mixed>(T, a.F, a.o));
+    L.finished = actorFinished<Rev, Sympy>(L, a, o);
   }
   if (L.finished || pathAbort(T, L.propLimit, o.surfaceTolerance)) return kPhaseFinished;
   if (L.nv.tSurf < 0) {
     T.cNav = kNotSet;
-    L.status = getNextTarget<Rev, Layers>(L.nv, T, geo, o, L.seq, layerCtx(a, L.q), -1);
+    L.status = getNextTarget<Rev, Layers>(L.nv, T, geo, a.o, L.seq, layerCtx(a, L.q), -1);
     if (L.status) return kPhaseFinished;
   }
   return kPhaseStepping;
@@ -509,7 +557,7 @@ __device__ inline int laneFilter(Lane& L, const FwdArgs& a, const DevSurface* ge
       }
     }
     if (L.status) return kPhaseFinished;
-    L.finished = actorFinished<Rev, Sympy>(L, a);
+    L.finished = actorFinished<Rev, Sympy>(L, a, o);
   }
   if (L.finished || pathAbort(T, L.propLimit, o.surfaceTolerance)) return kPhaseFinished;
   T.cNav = kNotSet;

@@ -62,15 +62,18 @@ __device__ inline float divRecipF(float a, float b, float y) {
   return fmaf(fmaf(-q, b, a), y, q);
 }
 
-// The FP32 copy of the map.  Fast: a cell-major copy and widths whose
-// reciprocals are normal numbers (DevField::recipF); otherwise point arrays
-// may be read and the axes divide.
-template <bool Fast>
+// The FP32 copy of the map: fast for a cell-major copy and widths whose
+// reciprocals are normal numbers (DevField::recipF); otherwise the axes
+// divide and point arrays may be read.
 struct MapFieldF {
   const DevField& F;
   CellCache c;
   __device__ inline bool operator()(const F3& p, F3& out) const {
     out = mkf(0.f, 0.f, 0.f);
+    return F.cellsF && F.recipF ? lookup<true>(p, out) : lookup<false>(p, out);
+  }
+  template <bool Fast>
+  __device__ inline bool lookup(const F3& p, F3& out) const {
     const float x[3] = {p.x, p.y, p.z};
     bool in = true;
 #pragma unroll
@@ -123,13 +126,14 @@ struct MapFieldF {
   }
 };
 
-template <typename Step>
-__device__ inline int withFieldF(const DevField& F, const CellCache& c, Step&& step) {
-  if (F.kind == ACTS_KF_FIELD_CONSTANT)
-    return step(UniformFieldF{mkf(static_cast<float>(F.B[0]), static_cast<float>(F.B[1]),
-                                  static_cast<float>(F.B[2]))});
-  if (F.cellsF && F.recipF) return step(MapFieldF<true>{F, c});
-  return step(MapFieldF<false>{F, c});
+__device__ inline int fieldAtF(const DevField& F, const F3& p, F3& out) {
+  if (F.kind == ACTS_KF_FIELD_CONSTANT) {
+    out = mkf(static_cast<float>(F.B[0]), static_cast<float>(F.B[1]), static_cast<float>(F.B[2]));
+    return 0;
+  }
+  return MapFieldF{F, CellCache{nullptr, nullptr, nullptr}}(p, out)
+             ? 0
+             : ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
 }
 
 __device__ inline float stepScalingF(float tol, float err) {

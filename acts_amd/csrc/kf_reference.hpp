@@ -217,7 +217,7 @@ __device__ inline void initializeFromBound(Track& T, const DevSurface& s, const 
 // Propagator::propagate(start, target) to the line in direction `direction`
 // with ForcedSurfaceReached + PathLimitReached (loop protection on);
 // returns a status, T holds the state at the end.
-template <bool Mixed, bool Sympy = false>
+template <bool Mixed, bool Sympy, bool Map>
 __device__ inline int propagateToLine(Track& T, const LineRef& L, const DevField& F,
                                       const CellCache& cache, const DevOpts& o,
                                       double direction) {
@@ -240,7 +240,7 @@ __device__ inline int propagateToLine(Track& T, const LineRef& L, const DevField
   };
   if (checkAbort()) return 0;
   for (uint32_t steps = 0; steps < o.maxSteps; ++steps) {
-    const int sst = stepTrack<Mixed, Sympy>(T, F, cache, o, direction, true);
+    const int sst = stepTrack<Mixed, Sympy, Map>(T, F, cache, o, direction, true);
     if (sst) return sst;
     T.cNav = kNotSet;
     T.cActor = kNotSet;
@@ -252,7 +252,7 @@ __device__ inline int propagateToLine(Track& T, const LineRef& L, const DevField
 // extrapolateTrackToReferenceSurface for track t (states in the scratch,
 // smoothed first/last measurement states in `ref`); returns a status and
 // writes the parameters and covariance on the line.
-template <bool Mixed, bool Sympy = false>
+template <bool Mixed, bool Sympy, bool Map>
 __device__ inline int extrapolateTrack(int64_t q, const DevScratch& sc, const double* ref,
                                        const DevSurface* geo, const DevField& F,
                                        const CellCache& cache, const DevOpts& o,
@@ -299,7 +299,7 @@ __device__ inline int extrapolateTrack(int64_t q, const DevScratch& sc, const do
   const double direction = distance >= 0 ? 1.0 : -1.0;
   Track T;
   initializeFromBound<Sympy>(T, geo[si(sc, k, kISurf, q)], p, p + 6, o);
-  if (const int st = propagateToLine<Mixed, Sympy>(T, L, F, cache, o, direction)) return st;
+  if (const int st = propagateToLine<Mixed, Sympy, Map>(T, L, F, cache, o, direction)) return st;
   return lineBoundState<Sympy>(T, L, o.surfaceTolerance, params, cov);
 }
 
