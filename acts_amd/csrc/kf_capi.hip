@@ -15,6 +15,7 @@
 #include "kf_field_host.hpp"
 #include "kf_reference.hpp"
 #include "kf_forward.hpp"
+#include "kf_host_copy.hpp"
 #include "kf_states.hpp"
 
 using namespace kf;
@@ -481,6 +482,7 @@ struct acts_kf_ctx {
   DevBuf refBuf;
   // staging for the host-buffer entry point
   DevBuf inBuf, outBuf;
+  HostCopy hostCopy;
   // device address of the static workspace on this context's device
   void* staticWs = nullptr;
 };
@@ -1344,18 +1346,40 @@ int acts_kf_fit_batch(acts_kf_ctx* c, const acts_kf_batch_in* in,
       {in->meas_indices, in->meas_indices ? sizeof(uint8_t) * 2 * nMeas : 0}};
   constexpr int nIn = sizeof(ins) / sizeof(ins[0]);
   auto al = [](size_t x) { return (x + 255) / 256 * 256; };
-  size_t total = 0;
-  for (const Sec& q : ins) total += al(q.bytes);
+  // pageable arrays go through the context's pinned memory, packed at the
+  // front of the block (under capture, or without pinned memory, the runtime
+  // copies them); the runtime copies all others (pinned: straight by DMA)
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  KF_HIP(hipStreamIsCapturing(s, &capture));
+  const bool canStage = capture == hipStreamCaptureStatusNone;
+  bool staged[nIn];
+  size_t total = 0, stagedBytes = 0;
+  for (int i = 0; i < nIn; ++i) {
+    staged[i] = canStage && ins[i].bytes && HostCopy::pageable(ins[i].src);
+    total += al(ins[i].bytes);
+    if (staged[i]) stagedBytes += al(ins[i].bytes);
+  }
+  if (!c->hostCopy.reserve(stagedBytes)) {
+    (void)hipGetLastError();
+    std::fill(staged, staged + nIn, false);
+    stagedBytes = 0;
+  }
   if (c->inBuf.ensure(total)) return fail(ACTS_KF_ERR_OUT_OF_MEMORY, "input staging alloc");
   char* base = static_cast<char*>(c->inBuf.p);
   void* dptr[nIn];
-  size_t off = 0;
+  CopyPiece inPieces[nIn];
+  int nInPieces = 0;
+  size_t packed = 0, off = stagedBytes;
   for (int i = 0; i < nIn; ++i) {
-    dptr[i] = base + off;
-    if (ins[i].bytes)
+    size_t& at = staged[i] ? packed : off;
+    dptr[i] = base + at;
+    if (staged[i])
+      inPieces[nInPieces++] = {static_cast<char*>(const_cast<void*>(ins[i].src)), at, ins[i].bytes};
+    else if (ins[i].bytes)
       KF_HIP(hipMemcpyAsync(dptr[i], ins[i].src, ins[i].bytes, hipMemcpyHostToDevice, s));
-    off += al(ins[i].bytes);
+    at += al(ins[i].bytes);
   }
+  KF_HIP(c->hostCopy.upload(inPieces, nInPieces, base, stagedBytes, c->device, s));
   acts_kf_batch_in din = *in;
   din.start_params = static_cast<const double*>(dptr[0]);
   din.start_cov = static_cast<const double*>(dptr[1]);
@@ -1392,16 +1416,32 @@ int acts_kf_fit_batch(acts_kf_ctx* c, const acts_kf_batch_in* in,
       {out->state_measurement, sizeof(int32_t) * nSeq},
       {out->reversed, sizeof(int32_t) * n}};
   constexpr int nOut = sizeof(outs) / sizeof(outs[0]);
-  size_t totalO = 0;
-  for (const OSec& q : outs)
-    if (q.host) totalO += al(q.bytes);
+  bool stagedO[nOut];
+  size_t totalO = 0, stagedBytesO = 0;
+  for (int i = 0; i < nOut; ++i) {
+    const size_t bytes = outs[i].host ? al(outs[i].bytes) : 0;
+    stagedO[i] = canStage && bytes && HostCopy::pageable(outs[i].host);
+    totalO += bytes;
+    if (stagedO[i]) stagedBytesO += bytes;
+  }
+  if (!c->hostCopy.reserve(stagedBytesO)) {
+    (void)hipGetLastError();
+    std::fill(stagedO, stagedO + nOut, false);
+    stagedBytesO = 0;
+  }
   if (c->outBuf.ensure(totalO)) return fail(ACTS_KF_ERR_OUT_OF_MEMORY, "output staging alloc");
   char* ob = static_cast<char*>(c->outBuf.p);
   void* optr[nOut];
-  off = 0;
+  CopyPiece outPieces[nOut];
+  int nOutPieces = 0;
+  packed = 0;
+  off = stagedBytesO;
   for (int i = 0; i < nOut; ++i) {
-    optr[i] = outs[i].host ? ob + off : nullptr;
-    if (outs[i].host) off += al(outs[i].bytes);
+    size_t& at = stagedO[i] ? packed : off;
+    optr[i] = outs[i].host ? ob + at : nullptr;
+    if (stagedO[i])
+      outPieces[nOutPieces++] = {static_cast<char*>(outs[i].host), at, outs[i].bytes};
+    if (outs[i].host) at += al(outs[i].bytes);
   }
   acts_kf_batch_out dout;
   dout.status = static_cast<int32_t*>(optr[0]);
@@ -1433,8 +1473,9 @@ int acts_kf_fit_batch(acts_kf_ctx* c, const acts_kf_batch_in* in,
   if (const int r = contextWorkspace(c, w, ws)) return r;
   if (const int r = launchFit(c, &din, &dout, s, w, ws, c->useGraph)) return r;
   for (int i = 0; i < nOut; ++i)
-    if (outs[i].host && outs[i].bytes)
+    if (outs[i].host && outs[i].bytes && !stagedO[i])
       KF_HIP(hipMemcpyAsync(outs[i].host, optr[i], outs[i].bytes, hipMemcpyDeviceToHost, s));
+  KF_HIP(c->hostCopy.download(outPieces, nOutPieces, ob, stagedBytesO, c->device, s));
   return markQueued(c, s);
 }
 
@@ -1532,6 +1573,7 @@ void acts_kf_destroy(acts_kf_ctx* c) {
   c->queueBuf.release();
   c->inBuf.release();
   c->outBuf.release();
+  c->hostCopy.release();
   if (c->geo) (void)hipFree(c->geo);
   if (c->slabs) (void)hipFree(c->slabs);
   if (c->fieldValues) (void)hipFree(c->fieldValues);
