@@ -178,15 +178,50 @@ constexpr int kSortBlock = 256;
 // momentum orders) a 500 000-track batch scans 0.12 M entries, not the 2 M
 // of one tile per 256 tracks (which took ~5 ms in one workgroup)
 constexpr int kSortTile = 4096;
-constexpr int kScanBlock = 1024;
 constexpr int kMaxKeys = 1026;  // lengths above 1023 share a bucket
 
 __device__ inline int64_t histIndex(int32_t key, int32_t nKeys, int64_t block, int64_t nBlocks) {
   return static_cast<int64_t>(nKeys - 1 - key) * nBlocks + block;
 }
 
-// The sort key of every track (its queue key, capped at kMaxKeys - 1),
-// once: a workgroup takes
+// The sort key of a track: its queue key, capped at kMaxKeys - 1.
+__device__ inline int32_t sortKey(const QueueKeyArgs& k, int64_t t, bool seam) {
+  int32_t key;
+  if (seam) {
+    key = k.byDirection ? kDirectionKeys
+          : k.byMomentum ? (kMomentumLenCap + 1) * kMomentumBins
+                         : k.maxLen + 1;
+  } else if (k.byDirection) {
+    key = directionKey(k, t);
+  } else {
+    const int32_t len = min(static_cast<int32_t>(k.seqOff[t + 1] - k.seqOff[t]), k.maxLen);
+    key = k.byMomentum ? momentumKey(k, t, len) : len;
+  }
+  return min(key, kMaxKeys - 1);
+}
+
+// Marks in `seam` the tracks (counted from off[0]'s) with a measurement m on
+// a cylinder near the seam; off[0..nt] are their measurement offsets.
+template <typename Offsets>
+__device__ inline void markSeam(const QueueKeyArgs& k, int64_t m, const Offsets& off, int nt,
+                                int32_t* seam) {
+  const int32_t s = k.measSurf[m];
+  if (s < 0 || s >= k.nSurfaces || k.geo[s].type != ACTS_KF_SURFACE_CYLINDER) return;
+  const double phi = k.measVal[2 * m] / k.geo[s].b0;
+  if (fabs(phi) > kPi - kSeamRisk) {
+    int lo = 0, hi = nt;  // off[lo] <= m < off[hi]
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) / 2;
+      if (off[mid] <= m)
+        lo = mid;
+      else
+        hi = mid;
+    }
+    seam[lo] = 1;
+  }
+}
+
+// The sort key of every track, once: a workgroup takes
 // kSortBlock consecutive tracks, reads their measurements with consecutive
 // threads on consecutive measurements (a thread per track walking its own
 // measurements touched a different cache line per lane and load and fetched
@@ -202,37 +237,11 @@ __global__ __launch_bounds__(kSortBlock) void queueKeyKernel(QueueKeyArgs k, int
   for (int i = threadIdx.x; i <= nt; i += kSortBlock) off[i] = k.measOff[t0 + i];
   seam[threadIdx.x] = 0;
   __syncthreads();
-  for (int64_t m = off[0] + threadIdx.x; m < off[nt]; m += kSortBlock) {
-    const int32_t s = k.measSurf[m];
-    if (s < 0 || s >= k.nSurfaces || k.geo[s].type != ACTS_KF_SURFACE_CYLINDER) continue;
-    const double phi = k.measVal[2 * m] / k.geo[s].b0;
-    if (fabs(phi) > kPi - kSeamRisk) {
-      int lo = 0, hi = nt;  // off[lo] <= m < off[hi]
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) / 2;
-        if (off[mid] <= m)
-          lo = mid;
-        else
-          hi = mid;
-      }
-      seam[lo] = 1;
-    }
-  }
+  for (int64_t m = off[0] + threadIdx.x; m < off[nt]; m += kSortBlock)
+    markSeam(k, m, off, nt, seam);
   __syncthreads();
   if (threadIdx.x >= nt) return;
-  const int64_t t = t0 + threadIdx.x;
-  int32_t key;
-  if (seam[threadIdx.x]) {
-    key = k.byDirection ? kDirectionKeys
-          : k.byMomentum ? (kMomentumLenCap + 1) * kMomentumBins
-                         : k.maxLen + 1;
-  } else if (k.byDirection) {
-    key = directionKey(k, t);
-  } else {
-    const int32_t len = min(static_cast<int32_t>(k.seqOff[t + 1] - k.seqOff[t]), k.maxLen);
-    key = k.byMomentum ? momentumKey(k, t, len) : len;
-  }
-  keys[t] = min(key, kMaxKeys - 1);
+  keys[t0 + threadIdx.x] = sortKey(k, t0 + threadIdx.x, seam[threadIdx.x] != 0);
 }
 
 __global__ __launch_bounds__(kSortBlock) void keyHistogramKernel(const int32_t* keys, int64_t n,
@@ -249,83 +258,58 @@ __global__ __launch_bounds__(kSortBlock) void keyHistogramKernel(const int32_t* 
     blockHist[histIndex(i, nKeys, blockIdx.x, gridDim.x)] = h[i];
 }
 
-// Exclusive prefix sum of `count` ints in place, one workgroup: each thread
-// sums a contiguous chunk, the chunk sums are scanned in LDS, each thread
-// rewrites its chunk.
-__global__ __launch_bounds__(kScanBlock) void exclusiveScanKernel(int32_t* a, int64_t count) {
-  __shared__ int32_t part[kScanBlock];
-  const int64_t chunk = (count + kScanBlock - 1) / kScanBlock;
-  const int64_t lo = threadIdx.x * chunk;
-  const int64_t hi = min(lo + chunk, count);
-  int32_t sum = 0;
-  for (int64_t i = lo; i < hi; ++i) sum += a[i];
-  part[threadIdx.x] = sum;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int32_t acc = 0;
-    for (int i = 0; i < kScanBlock; ++i) {
-      const int32_t c = part[i];
-      part[i] = acc;
-      acc += c;
-    }
+// Inclusive prefix sum over the workgroup of each thread's `v` (blockDim.x
+// threads, a multiple of 64; `waves` has an entry per wavefront).
+__device__ inline int32_t blockScan(int32_t v, int32_t* waves) {
+  const int lane = static_cast<int>(threadIdx.x) & 63, wave = static_cast<int>(threadIdx.x) >> 6;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int32_t u = __shfl_up(v, d);
+    v += lane >= d ? u : 0;
   }
+  if (lane == 63) waves[wave] = v;
   __syncthreads();
-  int32_t acc = part[threadIdx.x];
-  for (int64_t i = lo; i < hi; ++i) {
-    const int32_t c = a[i];
-    a[i] = acc;
-    acc += c;
-  }
+  for (int w = 0; w < wave; ++w) v += waves[w];
+  __syncthreads();
+  return v;
 }
 
-// The scan of the whole histogram array in three passes over chunks of
-// kScanChunk entries, so that many workgroups read it coalesced: the sum of
-// every chunk (chunkSumKernel), the exclusive scan of those sums
-// (exclusiveScanKernel, one workgroup over a few hundred entries), then each
-// chunk scanned in LDS from its sum's offset (chunkScanKernel).
+// The exclusive scan of the whole histogram array over chunks of kScanChunk
+// entries, so that many workgroups read it coalesced: with more than one
+// chunk the sum of every chunk (chunkSumKernel), then each chunk scanned in
+// its workgroup from the sums of the chunks before it.
 constexpr int kScanChunk = 4096;
 constexpr int kScanThreads = 256;
 __global__ __launch_bounds__(kScanThreads) void chunkSumKernel(const int32_t* a, int64_t count,
                                                                int32_t* sums) {
-  __shared__ int32_t red[kScanThreads];
+  __shared__ int32_t waves[kScanThreads / 64];
   const int64_t lo = static_cast<int64_t>(blockIdx.x) * kScanChunk;
   const int64_t hi = min<int64_t>(count, lo + kScanChunk);
   int32_t sum = 0;
   for (int64_t i = lo + threadIdx.x; i < hi; i += kScanThreads) sum += a[i];
-  red[threadIdx.x] = sum;
-  __syncthreads();
-  for (int w = kScanThreads / 2; w > 0; w >>= 1) {
-    if (static_cast<int>(threadIdx.x) < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) sums[blockIdx.x] = red[0];
+  sum = blockScan(sum, waves);
+  if (threadIdx.x == kScanThreads - 1) sums[blockIdx.x] = sum;
 }
 
 __global__ __launch_bounds__(kScanThreads) void chunkScanKernel(int32_t* a, int64_t count,
-                                                                const int32_t* offsets) {
+                                                                const int32_t* sums) {
   constexpr int kPer = kScanChunk / kScanThreads;
   __shared__ int32_t v[kScanChunk];
-  __shared__ int32_t part[kScanThreads];
+  __shared__ int32_t waves[kScanThreads / 64];
+  __shared__ int32_t before;
   const int64_t lo = static_cast<int64_t>(blockIdx.x) * kScanChunk;
   const int n = static_cast<int>(min<int64_t>(kScanChunk, count - lo));
+  int32_t part = 0;
+  for (int i = threadIdx.x; i < static_cast<int>(blockIdx.x); i += kScanThreads) part += sums[i];
+  part = blockScan(part, waves);
+  if (threadIdx.x == kScanThreads - 1) before = part;
   for (int i = threadIdx.x; i < n; i += kScanThreads) v[i] = a[lo + i];
   __syncthreads();
   const int first = static_cast<int>(threadIdx.x) * kPer;
   int32_t sum = 0;
   for (int j = 0; j < kPer; ++j)
     if (first + j < n) sum += v[first + j];
-  part[threadIdx.x] = sum;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int32_t acc = offsets[blockIdx.x];
-    for (int t = 0; t < kScanThreads; ++t) {
-      const int32_t c = part[t];
-      part[t] = acc;
-      acc += c;
-    }
-  }
-  __syncthreads();
-  int32_t acc = part[threadIdx.x];
+  int32_t acc = before + blockScan(sum, waves) - sum;
   for (int j = 0; j < kPer; ++j) {
     if (first + j < n) {
       const int32_t c = v[first + j];
@@ -337,11 +321,58 @@ __global__ __launch_bounds__(kScanThreads) void chunkScanKernel(int32_t* a, int6
   for (int i = threadIdx.x; i < n; i += kScanThreads) a[lo + i] = v[i];
 }
 
+// The whole sort of a small batch in one workgroup and one launch: keys,
+// histogram, scan and scatter in LDS, and the queue counter.  The six
+// launches of the general sort took ~45 us, of which 9 in the scan of the
+// chunk sums, against ~15 for this at its largest batch, where one CU's
+// reading of the measurements begins to show.
+constexpr int kSmallSort = 4096;
+constexpr int kSmallSortThreads = 1024;
+__global__ __launch_bounds__(kSmallSortThreads) void smallSortKernel(QueueKeyArgs k, int32_t n,
+                                                                     int32_t nKeys, int32_t* perm,
+                                                                     int32_t* queue) {
+  __shared__ int32_t key[kSmallSort];  // first the seam marks
+  __shared__ int32_t h[kMaxKeys];
+  __shared__ int32_t waves[kSmallSortThreads / 64];
+  const int tid = static_cast<int>(threadIdx.x);
+  if (tid == 0) *queue = 0;
+  for (int i = tid; i < n; i += kSmallSortThreads) key[i] = 0;
+  for (int i = tid; i < nKeys; i += kSmallSortThreads) h[i] = 0;
+  __syncthreads();
+  for (int64_t m = k.measOff[0] + tid; m < k.measOff[n]; m += kSmallSortThreads)
+    markSeam(k, m, k.measOff, n, key);
+  __syncthreads();
+  for (int t = tid; t < n; t += kSmallSortThreads) {
+    key[t] = sortKey(k, t, key[t] != 0);
+    atomicAdd(&h[key[t]], 1);
+  }
+  __syncthreads();
+  // the first place of every key, the largest key first
+  constexpr int kPer = (kMaxKeys + kSmallSortThreads - 1) / kSmallSortThreads;
+  int32_t c[kPer], sum = 0;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int i = tid * kPer + j;
+    c[j] = i < nKeys ? h[nKeys - 1 - i] : 0;
+    sum += c[j];
+  }
+  int32_t acc = blockScan(sum, waves) - sum;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int i = tid * kPer + j;
+    if (i < nKeys) h[nKeys - 1 - i] = acc;
+    acc += c[j];
+  }
+  __syncthreads();
+  for (int t = tid; t < n; t += kSmallSortThreads) perm[atomicAdd(&h[key[t]], 1)] = t;
+}
+
 __global__ __launch_bounds__(kSortBlock) void keyScatterKernel(const int32_t* keys, int64_t n,
                                                                int32_t nKeys,
                                                                const int32_t* blockOffset,
-                                                               int32_t* perm) {
+                                                               int32_t* perm, int32_t* queue) {
   __shared__ int32_t h[kMaxKeys];
+  if (blockIdx.x == 0 && threadIdx.x == 0) *queue = 0;
   for (int i = threadIdx.x; i < nKeys; i += kSortBlock) h[i] = 0;
   __syncthreads();
   const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kSortTile;
@@ -1114,23 +1145,30 @@ static int launchFit(acts_kf_ctx* c, const acts_kf_batch_in* in,
     qk.geo = c->geo;
     qk.nSurfaces = c->nSurfaces;
     qk.maxLen = states;
-    const unsigned nb = static_cast<unsigned>(sortBlocks);
-    const unsigned nbKey = static_cast<unsigned>((n + kSortBlock - 1) / kSortBlock);
-    // the keys after the permutation in the same buffer (workspaceSizes)
-    int32_t* keys = perm + n;
-    hipLaunchKernelGGL(queueKeyKernel, dim3(nbKey), dim3(kSortBlock), 0, stream, qk, n, keys);
-    hipLaunchKernelGGL(keyHistogramKernel, dim3(nb), dim3(kSortBlock), 0, stream, keys, n,
-                       nKeys, hist);
-    const int64_t count = static_cast<int64_t>(nKeys) * sortBlocks;
-    const int64_t chunks = (count + kScanChunk - 1) / kScanChunk;
-    int32_t* sums = hist + count;
-    hipLaunchKernelGGL(chunkSumKernel, dim3(static_cast<unsigned>(chunks)), dim3(kScanThreads), 0,
-                       stream, hist, count, sums);
-    hipLaunchKernelGGL(exclusiveScanKernel, dim3(1), dim3(kScanBlock), 0, stream, sums, chunks);
-    hipLaunchKernelGGL(chunkScanKernel, dim3(static_cast<unsigned>(chunks)), dim3(kScanThreads), 0,
-                       stream, hist, count, sums);
-    hipLaunchKernelGGL(keyScatterKernel, dim3(nb), dim3(kSortBlock), 0, stream, keys, n,
-                       nKeys, hist, perm);
+    if (n <= kSmallSort) {
+      hipLaunchKernelGGL(smallSortKernel, dim3(1), dim3(kSmallSortThreads), 0, stream, qk,
+                         static_cast<int32_t>(n), nKeys, perm, ws.queue);
+    } else {
+      const unsigned nb = static_cast<unsigned>(sortBlocks);
+      const unsigned nbKey = static_cast<unsigned>((n + kSortBlock - 1) / kSortBlock);
+      // the keys after the permutation in the same buffer (workspaceSizes)
+      int32_t* keys = perm + n;
+      hipLaunchKernelGGL(queueKeyKernel, dim3(nbKey), dim3(kSortBlock), 0, stream, qk, n, keys);
+      hipLaunchKernelGGL(keyHistogramKernel, dim3(nb), dim3(kSortBlock), 0, stream, keys, n,
+                         nKeys, hist);
+      const int64_t count = static_cast<int64_t>(nKeys) * sortBlocks;
+      const unsigned chunks = static_cast<unsigned>((count + kScanChunk - 1) / kScanChunk);
+      int32_t* sums = hist + count;
+      if (chunks > 1)
+        hipLaunchKernelGGL(chunkSumKernel, dim3(chunks), dim3(kScanThreads), 0, stream, hist, count,
+                           sums);
+      hipLaunchKernelGGL(chunkScanKernel, dim3(chunks), dim3(kScanThreads), 0, stream, hist, count,
+                         sums);
+      hipLaunchKernelGGL(keyScatterKernel, dim3(nb), dim3(kSortBlock), 0, stream, keys, n,
+                         nKeys, hist, perm, ws.queue);
+    }
+  } else {
+    hipLaunchKernelGGL(zeroKernel, dim3(1), dim3(64), 0, stream, ws.queue, 1);
   }
   FwdArgs fa;
   fa.in = b;
@@ -1154,7 +1192,6 @@ static int launchFit(acts_kf_ctx* c, const acts_kf_batch_in* in,
   fa.rv.rec = ws.rev;
   fa.rv.reached = ws.revReached;
   int32_t* queue = ws.queue;
-  hipLaunchKernelGGL(zeroKernel, dim3(1), dim3(64), 0, stream, queue, 1);
   const int64_t waves = std::min(blocks, c->residentWaves);
   if (timing) KF_HIP(hipEventRecord(c->ev[0], stream));
   hipLaunchKernelGGL(forwardKernel(c),
