@@ -284,12 +284,10 @@ __device__ inline double divBy(double a, double b, double y) {
 KF_HD V3 unit(const V3& a) {
 #ifdef __HIP_DEVICE_COMPILE__
   const double z = dot(a, a);
-  if (z > 0.0) {
-    const double n = sqrt(z);
-    const double y = 1.0 / n;
-    return mk(divBy(a.x, n, y), divBy(a.y, n, y), divBy(a.z, n, y));
-  }
-  return a;
+  const double n = sqrt(z);
+  const double y = 1.0 / n;
+  const V3 u = mk(divBy(a.x, n, y), divBy(a.y, n, y), divBy(a.z, n, y));
+  return z > 0.0 ? u : a;
 #else
   return normalized(a);
 #endif

@@ -143,6 +143,33 @@ KF_HD Isect intersect(const DevSurface& s, const V3& pos, const V3& dir, double 
   return intersect(surfaceLine(s), pos, dir, tol);
 }
 
+// Solution `idx` of intersect() in straight-line code, for the check after
+// every step: both kinds of surface computed and one selected (a wavefront
+// of barrel and disc tracks computes both anyway).  Returns whether there is
+// an intersection, on the surface if |path| < tol.
+__device__ inline bool intersectOne(const SurfaceLine& s, const V3& pos, const V3& dir, int idx,
+                                    double& path) {
+  const V3& ax = s.axis;
+  const V3 pcXcd = cross(mk(pos.x - s.t.x, pos.y - s.t.y, pos.z - s.t.z), ax);
+  const V3 ldXcd = cross(dir, ax);
+  const double a = dot(ldXcd, ldXcd);
+  const double b = 2. * dot(ldXcd, pcXcd);
+  const double c = dot(pcXcd, pcXcd) - (s.b0 * s.b0);
+  const double disc = b * b - 4 * a * c;
+  const double sq = sqrt(disc);
+  const double q = -0.5 * (b + (b > 0 ? sq : -sq));
+  const double first = q / a;
+  const double second = c / q;
+  const bool ordered = disc == 0 || first <= second;
+  const double other = disc == 0 ? first : second;
+  const double cyl = (idx != 0) == ordered ? other : first;
+  const double denom = dot(dir, ax);
+  const double plane = dot(ax, mk(s.t.x - pos.x, s.t.y - pos.y, s.t.z - pos.z)) / denom;
+  const bool isCyl = s.type == ACTS_KF_SURFACE_CYLINDER;
+  path = isCyl ? cyl : plane;
+  return isCyl ? disc >= 0 : !(denom == 0);
+}
+
 // The bounds check of Surface::intersect with BoundaryTolerance::None at
 // the intersection point x: full-azimuth cylinders compare the local z with
 // the half length plus the tolerance (CylinderSurface.cpp:242-257), full
@@ -456,16 +483,15 @@ struct MapField {
     out = mk(0.0, 0.0, 0.0);
     if (!(F.cells && F.recip)) return gridField(F, p, out) == 0;
     const double x[3] = {p.x, p.y, p.z};
+    // bin, lower edge and weight of each axis, as gridLocate; a point outside
+    // reads some cell of the map, and the caller drops the result
     bool in = true;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) in = in & (x[a] >= F.min[a]) & !(x[a] >= F.upper[a]);
-    if (!in) return false;
-    // bin, lower edge and weight of each axis, as gridLocate
     int lo[3];
     double f[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      const double u = divRecip(x[a] - F.min[a], F.width[a], F.rw[a]);
+      in = in & (x[a] >= F.min[a]) & !(x[a] >= F.upper[a]);
+      const double u = fmin(fmax(divRecip(x[a] - F.min[a], F.width[a], F.rw[a]), 0.0), 1e9);
       int bin = static_cast<int>(floor(u) + 1);
       bin = bin < 1 ? 1 : (bin > F.nb[a] ? F.nb[a] : bin);
       lo[a] = bin - 1;
@@ -475,10 +501,13 @@ struct MapField {
     // kMaxCellBytes keeps the cell index within 32 bits
     const int32_t cell = (lo[0] * F.nb[1] + lo[1]) * F.nb[2] + lo[2];
     double v[kCellValues];
-    if (c.idx && c.idx[0] == cell) {
+    bool hit = false;
+    if (c.idx) {
+      hit = c.idx[0] == cell;
 #pragma unroll
       for (int j = 0; j < kCellValues; ++j) v[j] = c.v[j * kCellCacheStride];
-    } else {
+    }
+    if (!hit) {
       const double* q = static_cast<const double*>(
           __builtin_assume_aligned(F.cells + static_cast<int64_t>(kCellDoubles) * cell, 64));
 #pragma unroll
@@ -500,7 +529,7 @@ struct MapField {
       for (int k = 0; k < 3; ++k) d[i][k] = (1 - f[1]) * e[2 * i][k] + f[1] * e[2 * i + 1][k];
     out = mk((1 - f[0]) * d[0][0] + f[0] * d[1][0], (1 - f[0]) * d[0][1] + f[0] * d[1][1],
              (1 - f[0]) * d[0][2] + f[0] * d[1][2]);
-    return true;
+    return in;
   }
 };
 
@@ -539,7 +568,7 @@ __device__ inline int rkTrials(const Track& T, const Field& field, const DevOpts
   const V3& pos = S.pos;
   const V3& dir = S.dir;
   const double qop = S.qop;
-  if (!field(pos, S.B1)) return ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
+  const bool insideHere = field(pos, S.B1);
   const V3 c1 = cross(dir, S.B1);
   S.k1 = mk(qop * c1.x, qop * c1.y, qop * c1.z);
   const V3& k1 = S.k1;
@@ -549,8 +578,7 @@ __device__ inline int rkTrials(const Track& T, const Field& field, const DevOpts
   double h2, half_h, err;
   int nTrials = 0;
   int status = 0;
-  bool again;
-  do {
+  while (true) {
     ++nTrials;
     h2 = h * h;
     half_h = h * 0.5;
@@ -558,9 +586,9 @@ __device__ inline int rkTrials(const Track& T, const Field& field, const DevOpts
     const V3 p1 = mk((pos.x + half_h * dir.x) + h28 * k1.x,
                      (pos.y + half_h * dir.y) + h28 * k1.y,
                      (pos.z + half_h * dir.z) + h28 * k1.z);
-    // a lookup outside the map ends the step below; what is computed in
-    // between is not used
-    bool inside = field(p1, S.B2);
+    // a lookup outside the map ends the step below; what is computed with
+    // it is not used
+    bool inside = field(p1, S.B2) & insideHere;
     S.k2 = kEval(qop, dir, half_h, k1, S.B2);
     S.k3 = kEval(qop, dir, half_h, S.k2, S.B2);
     const double h22 = h2 * 0.5;
@@ -574,17 +602,15 @@ __device__ inline int rkTrials(const Track& T, const Field& field, const DevOpts
     const double e2 = ((k1.z - S.k2.z) - S.k3.z) + S.k4.z;
     err = h2 * ((fabs(e0) + fabs(e1)) + fabs(e2));
     err = fmax(1e-20, err);
-    again = inside && !(err <= 4.0 * o.stepTolerance);
-    if (again) {
-      h *= stepScaling(o.stepTolerance, err);
-      if (fabs(h) < fabs(o.stepSizeCutOff))
-        status = ACTS_KF_STATUS_STEP_SIZE_STALLED;
-      else if (static_cast<uint32_t>(nTrials) > o.maxTrials)
-        status = ACTS_KF_STATUS_STEP_ADJUSTMENT_FAILED;
-      again = status == 0;
-    }
-    if (!inside) status = ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
-  } while (again);
+    status = inside ? 0 : ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
+    if (!inside || err <= 4.0 * o.stepTolerance) break;
+    h *= stepScaling(o.stepTolerance, err);
+    status = fabs(h) < fabs(o.stepSizeCutOff) ? ACTS_KF_STATUS_STEP_SIZE_STALLED
+             : static_cast<uint32_t>(nTrials) > o.maxTrials
+                 ? ACTS_KF_STATUS_STEP_ADJUSTMENT_FAILED
+                 : 0;
+    if (status) break;
+  }
   S.h = h;
   S.h2 = h2;
   S.half_h = half_h;
@@ -835,14 +861,13 @@ __device__ inline int rkStepSympy(Track& T, const Field& field, const DevOpts& o
   const double qop = T.qop;
   const double m = o.mass;
   V3 B1;
-  if (!field(pos, B1)) return ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
+  const bool insideHere = field(pos, B1);
   const double initialH = stepValue(T) * propDir;
   double h = initialH, err = 0, hThird = 0;
   int nTrials = 0;
   V3 bend1, bend2, bend3, kick1, dir2, dir3, dir4, dirEnd, kick4;
   int status = 0;
-  bool again;
-  do {
+  while (true) {
     ++nTrials;
     const double halfHQop = h * qop / 2;
     hThird = divBy(h, 3.0, 1.0 / 3.0);
@@ -853,7 +878,7 @@ __device__ inline int rkStepSympy(Track& T, const Field& field, const DevOpts& o
     const V3 dirHalfSum = add3(dir2, dir);
     const V3 pos2 = add3(pos, scale3(hQuarter, dirHalfSum));
     V3 B2;
-    bool inside = field(pos2, B2);
+    bool inside = field(pos2, B2) & insideHere;
     bend2 = scale3(halfHQop, B2);
     dir3 = add3(dir, cross(dir2, bend2));
     dir4 = add3(dir, cross(dir3, bend2));
@@ -867,17 +892,15 @@ __device__ inline int rkStepSympy(Track& T, const Field& field, const DevOpts& o
     err = 2 * fabs(h) * ((fabs(e.x) + fabs(e.y)) + fabs(e.z));
     const bool ok = !(err > 4.0 * o.stepTolerance);
     err = fmax(1e-20, err);
-    again = inside && !ok;
-    if (again) {
-      h *= stepScaling(o.stepTolerance, err);
-      if (fabs(h) < fabs(o.stepSizeCutOff))
-        status = ACTS_KF_STATUS_STEP_SIZE_STALLED;
-      else if (static_cast<uint32_t>(nTrials) > o.maxTrials)
-        status = ACTS_KF_STATUS_STEP_ADJUSTMENT_FAILED;
-      again = status == 0;
-    }
-    if (!inside) status = ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
-  } while (again);
+    status = inside ? 0 : ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
+    if (!inside || ok) break;
+    h *= stepScaling(o.stepTolerance, err);
+    status = fabs(h) < fabs(o.stepSizeCutOff) ? ACTS_KF_STATUS_STEP_SIZE_STALLED
+             : static_cast<uint32_t>(nTrials) > o.maxTrials
+                 ? ACTS_KF_STATUS_STEP_ADJUSTMENT_FAILED
+                 : 0;
+    if (status) break;
+  }
   if (status) return status;
   const V3 newPos = add3(pos, scale3(hThird, add3(add3(dir2, dir3), dir4)));
   const V3 newDirX3 = add3(scale3(2, dir3), add3(add3(kick1, dirEnd), kick4));

@@ -985,9 +985,9 @@ __device__ inline int stepTrack(Track& T, const DevField& F, const CellCache& ca
 // PathLimitReached::checkAbort (StandardAborters.hpp:41-61)
 __device__ inline bool pathAbort(Track& T, double limit, double tol) {
   const double distance = fabs(limit) - fabs(T.pathAcc);
-  if (fabs(distance) < fabs(tol)) return true;
-  updateStep(T.cActor, distance);
-  return false;
+  const bool abort = fabs(distance) < fabs(tol);
+  T.cActor = !abort & (fabs(distance) < fabs(T.cActor)) ? distance : T.cActor;
+  return abort;
 }
 
 }  // namespace kf

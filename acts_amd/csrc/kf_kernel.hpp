@@ -330,19 +330,21 @@ __device__ inline int laneStep(Lane& L, const FwdArgs& a, const StepArgs& s,
                                const DevSurface* geo, const CellCache& cache) {
   const DevOpts& o = s.o;
   Track& T = L.T;
-  // the target's geometry for the intersection after the step, read before
-  // it, so that the step's arithmetic covers the wait
-  const SurfaceLine target = surfaceLine(geo[L.nv.tSurf >= 0 ? L.nv.tSurf : 0]);
-  if (L.iter >= o.maxSteps) {
-    L.status = ACTS_KF_STATUS_STEP_COUNT_LIMIT;
-    return kPhaseFinished;
-  }
-  constexpr double propDir = Rev ? -1.0 : 1.0;
-  if (!Rev && s.skipAfter > 0 && !L.noTransport && !L.replaying && !L.noSkip &&
-      L.iter - L.lastSurfIter >= static_cast<uint32_t>(s.skipAfter)) {
+  const bool atLimit = L.iter >= o.maxSteps;
+  const bool startSkip = !Rev & (s.skipAfter > 0) & !L.noTransport & !L.replaying & !L.noSkip &
+                         (L.iter - L.lastSurfIter >= static_cast<uint32_t>(s.skipAfter));
+  if (atLimit | startSkip) {
+    if (atLimit) {
+      L.status = ACTS_KF_STATUS_STEP_COUNT_LIMIT;
+      return kPhaseFinished;
+    }
     a.ckpt[static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x] = L;
     L.noTransport = true;
   }
+  constexpr double propDir = Rev ? -1.0 : 1.0;
+  // the target's geometry for the intersection after the step, read before
+  // it, so that the step's arithmetic covers the wait
+  const SurfaceLine target = surfaceLine(geo[L.nv.tSurf >= 0 ? L.nv.tSurf : 0]);
   ++L.iter;
   const bool transport = !L.noTransport && !pastLastSurface<Rev>(L);
   const int sst = stepTrack<Mixed, Sympy, Map>(T, s.F, cache, o, propDir, transport);
@@ -357,8 +359,8 @@ __device__ inline int laneStep(Lane& L, const FwdArgs& a, const StepArgs& s,
 // measurements handled, the path limit, and for the reverse filter its
 // target (each check updates the actor step size, in this order).
 template <bool Rev, bool Sympy>
-__device__ inline bool actorFinished(Lane& L, const FwdArgs& a, const DevOpts& o) {
-  bool fin = (L.nMeasStates == L.nUnique) || pathAbort(L.T, L.kfLimit, o.surfaceTolerance);
+__device__ inline bool actorFinished(Lane& L, const FwdArgs& a) {
+  bool fin = (L.nMeasStates == L.nUnique) || pathAbort(L.T, L.kfLimit, a.o.surfaceTolerance);
   if constexpr (Rev) {
     if (a.rv.hasTarget) fin = reverseTargetReached<Sympy>(L, a) || fin;
   }
@@ -373,29 +375,47 @@ __device__ inline int laneAfterStep(Lane& L, const FwdArgs& a, const DevOpts& o,
   Track& T = L.T;
   T.cNav = kNotSet;
   T.cActor = kNotSet;
-  if (L.nv.tSurf >= 0) {
-    Isect x;
-    if constexpr (Layers)
-      x = targetIntersection<Rev, true>(T, geo[L.nv.tSurf], o);
-    else
-      x = intersect(target, T.pos, navDir<Rev>(T), o.surfaceTolerance);
-    const int ps = updateSurfaceStatus<Rev>(T, x, L.nv.tIdx);
-    if (ps == kOnSurface && !L.nv.navBreak) L.reached = L.nv.tSurf;
-    if (ps != kReachable) L.nv.tSurf = -1;
+  // Selects instead of branches where they are cheap: a branch costs a
+  // wavefront ~30 cycles, the ~44 of a step in a uniform field a fifth of it.
+  const bool hasTarget = L.nv.tSurf >= 0;
+  bool on, reachable;
+  if constexpr (Layers) {
+    on = reachable = false;
+    if (hasTarget) {
+      const int ps =
+          updateSurfaceStatus<Rev>(T, targetIntersection<Rev, true>(T, geo[L.nv.tSurf], o),
+                                   L.nv.tIdx);
+      on = ps == kOnSurface;
+      reachable = ps == kReachable;
+    }
+  } else {
+    // updateSingleSurfaceStatus (updateSurfaceStatus)
+    double path;
+    const bool meets = intersectOne(target, T.pos, navDir<Rev>(T), L.nv.tIdx, path) & hasTarget;
+    on = meets & (fabs(path) < fabs(o.surfaceTolerance));
+    reachable = meets & !on & (path > -DBL_MAX) & (path < DBL_MAX + kOnSurfaceTolerance);
+    T.cNav = (on | reachable) & (fabs(path) < kNotSet) ? path : kNotSet;
   }
-  if (L.reached >= 0) return kPhaseSurface;
-  // act without a current surface: only the finalisation checks
-  if (!L.finished) {
-    if (L.kfLimit == DBL_MAX) limitPath(L.kfLimit, loopLimit<Mixed>(T, a.F, a.o));
-    L.finished = actorFinished<Rev, Sympy>(L, a, o);
+  L.reached = on & !L.nv.navBreak ? L.nv.tSurf : L.reached;
+  L.nv.tSurf = reachable ? L.nv.tSurf : -1;
+  // act without a current surface: only the finalisation checks (on a
+  // surface they come after the filter; that they have lowered the actor
+  // step size to the same distances before makes no difference)
+  const bool open = L.reached < 0;
+  if (open & (L.kfLimit == DBL_MAX)) limitPath(L.kfLimit, loopLimit<Mixed>(T, a.F, a.o));
+  bool fin = pathAbort(T, L.kfLimit, o.surfaceTolerance) | (L.nMeasStates == L.nUnique);
+  if constexpr (Rev) {
+    if (open && a.rv.hasTarget) fin = reverseTargetReached<Sympy>(L, a) || fin;
   }
-  if (L.finished || pathAbort(T, L.propLimit, o.surfaceTolerance)) return kPhaseFinished;
-  if (L.nv.tSurf < 0) {
+  L.finished = open & fin;
+  const bool end = pathAbort(T, L.propLimit, o.surfaceTolerance) | fin;
+  int phase = open ? (end ? kPhaseFinished : kPhaseStepping) : kPhaseSurface;
+  if ((phase == kPhaseStepping) & (L.nv.tSurf < 0)) {
     T.cNav = kNotSet;
     L.status = getNextTarget<Rev, Layers>(L.nv, T, geo, a.o, L.seq, layerCtx(a, L.q), -1);
-    if (L.status) return kPhaseFinished;
+    phase = L.status ? kPhaseFinished : kPhaseStepping;
   }
-  return kPhaseStepping;
+  return phase;
 }
 
 // KalmanFitter::Actor::filter on the reached surface (KalmanFitter.hpp:
@@ -557,7 +577,7 @@ __device__ inline int laneFilter(Lane& L, const FwdArgs& a, const DevSurface* ge
       }
     }
     if (L.status) return kPhaseFinished;
-    L.finished = actorFinished<Rev, Sympy>(L, a, o);
+    L.finished = actorFinished<Rev, Sympy>(L, a);
   }
   if (L.finished || pathAbort(T, L.propLimit, o.surfaceTolerance)) return kPhaseFinished;
   T.cNav = kNotSet;

@@ -75,16 +75,16 @@ struct MapFieldF {
   template <bool Fast>
   __device__ inline bool lookup(const F3& p, F3& out) const {
     const float x[3] = {p.x, p.y, p.z};
+    // a point outside reads some cell, and the caller drops the result
     bool in = true;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) in = in & (x[a] >= F.minF[a]) & !(x[a] >= F.upperF[a]);
-    if (!in) return false;
     int lo[3];
     float f[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       const float mn = F.minF[a], w = F.widthF[a];
-      const float u = Fast ? divRecipF(x[a] - mn, w, F.rwF[a]) : (x[a] - mn) / w;
+      in = in & (x[a] >= mn) & !(x[a] >= F.upperF[a]);
+      const float u =
+          fminf(fmaxf(Fast ? divRecipF(x[a] - mn, w, F.rwF[a]) : (x[a] - mn) / w, 0.f), 1e9f);
       int bin = static_cast<int>(floorf(u) + 1.f);
       bin = bin < 1 ? 1 : (bin > F.nb[a] ? F.nb[a] : bin);
       lo[a] = bin - 1;
@@ -96,10 +96,13 @@ struct MapFieldF {
       // the cell's record, one 128-byte line; kMaxCellBytes keeps its index
       // within 32 bits
       const int32_t cell = (lo[0] * F.nb[1] + lo[1]) * F.nb[2] + lo[2];
-      if (c.idx && c.idx[0] == cell) {
+      bool hit = false;
+      if (c.idx) {
+        hit = c.idx[0] == cell;
 #pragma unroll
         for (int j = 0; j < kCellValues; ++j) v[j] = c.vf[j * kCellCacheStride];
-      } else {
+      }
+      if (!hit) {
         const float* q = static_cast<const float*>(
             __builtin_assume_aligned(F.cellsF + static_cast<int64_t>(kCellFloats) * cell, 128));
 #pragma unroll
@@ -122,7 +125,7 @@ struct MapFieldF {
       }
     }
     out = interpolateF(v, f);
-    return true;
+    return in;
   }
 };
 
@@ -150,7 +153,7 @@ __device__ inline int rkStepMixed(Track& T, const Field& field, const DevOpts& o
   const float qop = static_cast<float>(T.qop);
   const float tol = static_cast<float>(o.stepTolerance);
   F3 B1;
-  if (!field(pos, B1)) return ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
+  const bool insideHere = field(pos, B1);
   const F3 c1 = crossf(dir, B1);
   const F3 k1 = mkf(qop * c1.x, qop * c1.y, qop * c1.z);
 
@@ -163,15 +166,14 @@ __device__ inline int rkStepMixed(Track& T, const Field& field, const DevOpts& o
   F3 B2, B3, k2, k3, k4;
   int nTrials = 0;
   int status = 0;
-  bool again;
-  do {
+  while (true) {
     ++nTrials;
     h2 = h * h;
     half_h = h * 0.5f;
     const float h28 = h2 * 0.125f;
     const F3 p1 = mkf((pos.x + half_h * dir.x) + h28 * k1.x, (pos.y + half_h * dir.y) + h28 * k1.y,
                       (pos.z + half_h * dir.z) + h28 * k1.z);
-    bool inside = field(p1, B2);
+    bool inside = field(p1, B2) & insideHere;
     F3 a = crossf(mkf(dir.x + half_h * k1.x, dir.y + half_h * k1.y, dir.z + half_h * k1.z), B2);
     k2 = mkf(qop * a.x, qop * a.y, qop * a.z);
     a = crossf(mkf(dir.x + half_h * k2.x, dir.y + half_h * k2.y, dir.z + half_h * k2.z), B2);
@@ -187,18 +189,16 @@ __device__ inline int rkStepMixed(Track& T, const Field& field, const DevOpts& o
     const float e2 = ((k1.z - k2.z) - k3.z) + k4.z;
     err = h2 * ((fabsf(e0) + fabsf(e1)) + fabsf(e2));
     err = fmaxf(1e-20f, err);
-    again = inside && !(err <= 4.0f * tol);
-    if (again) {
-      h *= stepScalingF(tol, err);
-      hD = static_cast<double>(h);
-      if (fabs(hD) < fabs(o.stepSizeCutOff))
-        status = ACTS_KF_STATUS_STEP_SIZE_STALLED;
-      else if (static_cast<uint32_t>(nTrials) > o.maxTrials)
-        status = ACTS_KF_STATUS_STEP_ADJUSTMENT_FAILED;
-      again = status == 0;
-    }
-    if (!inside) status = ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
-  } while (again);
+    status = inside ? 0 : ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
+    if (!inside || err <= 4.0f * tol) break;
+    h *= stepScalingF(tol, err);
+    hD = static_cast<double>(h);
+    status = fabs(hD) < fabs(o.stepSizeCutOff) ? ACTS_KF_STATUS_STEP_SIZE_STALLED
+             : static_cast<uint32_t>(nTrials) > o.maxTrials
+                 ? ACTS_KF_STATUS_STEP_ADJUSTMENT_FAILED
+                 : 0;
+    if (status) break;
+  }
   if (status) return status;
 
   // time and its derivatives in double (as rkTime): the time is not
@@ -346,7 +346,7 @@ __device__ inline int rkStepSympyMixed(Track& T, const Field& field, const DevOp
   const float qop = static_cast<float>(T.qop);
   const float tol = static_cast<float>(o.stepTolerance);
   F3 B1;
-  if (!field(pos, B1)) return ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
+  const bool insideHere = field(pos, B1);
   const double initialH = stepValue(T) * propDir;
   double hD = initialH;
   float h = static_cast<float>(initialH);
@@ -354,8 +354,7 @@ __device__ inline int rkStepSympyMixed(Track& T, const Field& field, const DevOp
   F3 bend1, bend2, bend3, kick1, c2, c3, kick4, dir2, dir3, dirEnd;
   int nTrials = 0;
   int status = 0;
-  bool again;
-  do {
+  while (true) {
     ++nTrials;
     const float halfHQop = h * qop * 0.5f;
     hThird = h / 3.f;
@@ -365,7 +364,7 @@ __device__ inline int rkStepSympyMixed(Track& T, const Field& field, const DevOp
     dir2 = add(dir, kick1);
     const F3 pos2 = add(pos, scl(hQuarter, add(dir2, dir)));
     F3 B2;
-    bool inside = field(pos2, B2);
+    bool inside = field(pos2, B2) & insideHere;
     bend2 = scl(halfHQop, B2);
     c2 = crossf(dir2, bend2);
     dir3 = add(dir, c2);
@@ -380,18 +379,16 @@ __device__ inline int rkStepSympyMixed(Track& T, const Field& field, const DevOp
     const F3 e = add(sub(sub(kick1, c2), c3), kick4);
     err = 2.f * fabsf(h) * ((fabsf(e.x) + fabsf(e.y)) + fabsf(e.z));
     err = fmaxf(1e-20f, err);
-    again = inside && !(err <= 4.0f * tol);
-    if (again) {
-      h *= stepScalingF(tol, err);
-      hD = static_cast<double>(h);
-      if (fabs(hD) < fabs(o.stepSizeCutOff))
-        status = ACTS_KF_STATUS_STEP_SIZE_STALLED;
-      else if (static_cast<uint32_t>(nTrials) > o.maxTrials)
-        status = ACTS_KF_STATUS_STEP_ADJUSTMENT_FAILED;
-      again = status == 0;
-    }
-    if (!inside) status = ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
-  } while (again);
+    status = inside ? 0 : ACTS_KF_STATUS_FIELD_OUT_OF_BOUNDS;
+    if (!inside || err <= 4.0f * tol) break;
+    h *= stepScalingF(tol, err);
+    hD = static_cast<double>(h);
+    status = fabs(hD) < fabs(o.stepSizeCutOff) ? ACTS_KF_STATUS_STEP_SIZE_STALLED
+             : static_cast<uint32_t>(nTrials) > o.maxTrials
+                 ? ACTS_KF_STATUS_STEP_ADJUSTMENT_FAILED
+                 : 0;
+    if (status) break;
+  }
   if (status) return status;
   const float m = o.mass;
   const double dtds = T.dtds;
