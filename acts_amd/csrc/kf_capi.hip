@@ -113,6 +113,26 @@ __global__ void zeroKernel(int32_t* p, int32_t count) {
   if (i < count) p[i] = 0;
 }
 
+// Queue place of sorted place i: the nSeam first tracks (the ones that may
+// become loopers) `spacing` places apart over the first `window` places, the
+// others between them.  In one block they filled the first wavefronts, where
+// loopers with different targets and step lengths took each other's steps
+// too (a step of several in the field map 3.2 to 3.8 against 2.4 thousand
+// x 4 cycles of one alone), which sets the length of a fit that is over
+// before its loopers: forward kernel of 5 000 field-map tracks 4.6 -> 4.2
+// ms, 100 000 7.1 -> 5.6, 200 000 7.2 -> 6.0.  A larger batch keeps the
+// block (window 1): few wavefronts then stay behind in quarantine with
+// their loopers while the others fit the rest (500 000: 6.7, spread 7.7 ms).
+constexpr int64_t kSpreadBatch = 4;  // batches, in resident lanes, to spread
+__device__ inline int32_t spreadPlace(int32_t i, int32_t nSeam, int32_t window) {
+  const int32_t spacing = nSeam > 0 ? min(64, window / nSeam) : 0;
+  if (spacing <= 1) return i;
+  const int32_t j = i - nSeam;
+  if (j < 0) return i * spacing;
+  if (j < nSeam * (spacing - 1)) return j / (spacing - 1) * spacing + 1 + j % (spacing - 1);
+  return i;
+}
+
 // Counting sort of the tracks by sequence length, longest first.
 // Queue key of a track: its sequence length (longest tracks first), or
 // maxLen + 1 for a track with a measurement within kSeamRisk rad of the +-pi
@@ -330,7 +350,7 @@ constexpr int kSmallSort = 4096;
 constexpr int kSmallSortThreads = 1024;
 __global__ __launch_bounds__(kSmallSortThreads) void smallSortKernel(QueueKeyArgs k, int32_t n,
                                                                      int32_t nKeys, int32_t* perm,
-                                                                     int32_t* queue) {
+                                                                     int32_t* queue, int32_t window) {
   __shared__ int32_t key[kSmallSort];  // first the seam marks
   __shared__ int32_t h[kMaxKeys];
   __shared__ int32_t waves[kSmallSortThreads / 64];
@@ -364,13 +384,18 @@ __global__ __launch_bounds__(kSmallSortThreads) void smallSortKernel(QueueKeyArg
     acc += c[j];
   }
   __syncthreads();
-  for (int t = tid; t < n; t += kSmallSortThreads) perm[atomicAdd(&h[key[t]], 1)] = t;
+  const int32_t nSeam = h[nKeys - 2];
+  __syncthreads();
+  for (int t = tid; t < n; t += kSmallSortThreads)
+    perm[spreadPlace(atomicAdd(&h[key[t]], 1), nSeam, window)] = t;
 }
 
 __global__ __launch_bounds__(kSortBlock) void keyScatterKernel(const int32_t* keys, int64_t n,
                                                                int32_t nKeys,
                                                                const int32_t* blockOffset,
-                                                               int32_t* perm, int32_t* queue) {
+                                                               int32_t* perm, int32_t* queue,
+                                                               int32_t window) {
+  const int32_t nSeam = blockOffset[histIndex(nKeys - 2, nKeys, 0, gridDim.x)];
   __shared__ int32_t h[kMaxKeys];
   if (blockIdx.x == 0 && threadIdx.x == 0) *queue = 0;
   for (int i = threadIdx.x; i < nKeys; i += kSortBlock) h[i] = 0;
@@ -380,8 +405,8 @@ __global__ __launch_bounds__(kSortBlock) void keyScatterKernel(const int32_t* ke
   for (int64_t t = t0 + threadIdx.x; t < t1; t += kSortBlock) {
     const int32_t key = keys[t];
     const int32_t rank = atomicAdd(&h[key], 1);
-    perm[blockOffset[histIndex(key, nKeys, blockIdx.x, gridDim.x)] + rank] =
-        static_cast<int32_t>(t);
+    perm[spreadPlace(blockOffset[histIndex(key, nKeys, blockIdx.x, gridDim.x)] + rank, nSeam,
+                     window)] = static_cast<int32_t>(t);
   }
 }
 
@@ -1145,9 +1170,12 @@ static int launchFit(acts_kf_ctx* c, const acts_kf_batch_in* in,
     qk.geo = c->geo;
     qk.nSurfaces = c->nSurfaces;
     qk.maxLen = states;
+    const int64_t lanes = c->residentWaves * kBlock;
+    const int32_t window =
+        n <= kSpreadBatch * lanes ? static_cast<int32_t>(std::min<int64_t>(n, lanes)) : 1;
     if (n <= kSmallSort) {
       hipLaunchKernelGGL(smallSortKernel, dim3(1), dim3(kSmallSortThreads), 0, stream, qk,
-                         static_cast<int32_t>(n), nKeys, perm, ws.queue);
+                         static_cast<int32_t>(n), nKeys, perm, ws.queue, window);
     } else {
       const unsigned nb = static_cast<unsigned>(sortBlocks);
       const unsigned nbKey = static_cast<unsigned>((n + kSortBlock - 1) / kSortBlock);
@@ -1165,7 +1193,7 @@ static int launchFit(acts_kf_ctx* c, const acts_kf_batch_in* in,
       hipLaunchKernelGGL(chunkScanKernel, dim3(chunks), dim3(kScanThreads), 0, stream, hist, count,
                          sums);
       hipLaunchKernelGGL(keyScatterKernel, dim3(nb), dim3(kSortBlock), 0, stream, keys, n,
-                         nKeys, hist, perm, ws.queue);
+                         nKeys, hist, perm, ws.queue, window);
     }
   } else {
     hipLaunchKernelGGL(zeroKernel, dim3(1), dim3(64), 0, stream, ws.queue, 1);
