@@ -13,9 +13,9 @@ a fit, never its results (acts_kf_options):
                      steps takes no new tracks until it ends;
   sched_transport_skip_steps  steps since the last surface after which a
                      track steps without the jacobian transport (helps
-                     where loopers never reach another surface, as with
-                     outliers that end at the loop-protection limit; hurts
-                     where tracks do reach one, as in the field map).
+                     where loopers never reach another surface, as in
+                     a uniform field; hurts where tracks do reach one, as
+                     in the field map).
 `autotune` times candidate settings on a device-resident sample of the
 workload by coordinate descent and keeps the fastest; results are cached in
 a JSON file keyed by the workload's shape.
@@ -42,7 +42,7 @@ SPACE = {
     "sched_wait_64ths": [16, 32, 48, 64],
     "length_sorted": [1, 0, 2, 3],
     "sched_quarantine_steps": [0, 100, 200, 400, -1],
-    "sched_transport_skip_steps": [0, 64, 256],
+    "sched_transport_skip_steps": [0, 64, -1],
 }
 DEFAULTS = {"sched_inner_steps": 16, "sched_wait_64ths": 64, "length_sorted": 1,
             "sched_quarantine_steps": 0, "sched_transport_skip_steps": 0}

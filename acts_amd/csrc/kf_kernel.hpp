@@ -332,6 +332,7 @@ __device__ inline int laneStep(Lane& L, const FwdArgs& a, const StepArgs& s,
   Track& T = L.T;
   const bool atLimit = L.iter >= o.maxSteps;
   const bool startSkip = !Rev & (s.skipAfter > 0) & !L.noTransport & !L.replaying & !L.noSkip &
+                         !pastLastSurface<Rev>(L) &
                          (L.iter - L.lastSurfIter >= static_cast<uint32_t>(s.skipAfter));
   if (atLimit | startSkip) {
     if (atLimit) {

@@ -56,7 +56,7 @@ class KalmanFitterOptions:
     sched_quarantine_steps: int = 0         # 0 = library default, < 0 = off
     kernel_timing: bool = False             # events around the kernels
     use_graph: bool = False                 # replay fits as a captured hipGraph
-    sched_transport_skip_steps: int = 0     # 0 = off
+    sched_transport_skip_steps: int = 0     # 0 = library default, < 0 = off
     # capi.NAVIGATOR_DIRECT: each track's given surface sequence
     # (DirectNavigator); capi.NAVIGATOR_LAYERS: the surfaces found from the
     # geometry (Navigator), the sequence offsets giving each track's slots

@@ -267,9 +267,12 @@ typedef struct acts_kf_options {
    * surface after all, it goes back to the saved state and repeats those
    * steps with the transport, so the results do not depend on it (a track
    * that never reaches another surface, e.g. a looper that ends at
-   * max_steps, uses no transport).  0 = off (default): a track that does
-   * reach a surface repeats the skipped steps, which costs more than the
-   * loopers save in the field map.  No reference counterpart.               */
+   * max_steps, uses no transport).  0 = the default: 200 steps in a uniform
+   * field; off in a field map, where loopers come back to a surface, repeat
+   * the skipped steps and lose more than they save.  Negative = off; always
+   * off with the layer navigator.  The saved states take up to 52 MB of
+   * device memory, grown with the batch; where they cannot be allocated the
+   * fit runs without.  No reference counterpart.                            */
   int32_t sched_transport_skip_steps;
   /* ACTS_KF_NAVIGATOR_* (default DIRECT)                                    */
   int32_t navigator;
