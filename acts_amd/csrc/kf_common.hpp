@@ -292,6 +292,23 @@ KF_HD V3 unit(const V3& a) {
   return normalized(a);
 #endif
 }
+// Sine and cosine of one angle: the values sin and cos give, from one argument
+// reduction.
+KF_HD void sinCos(double x, double& s, double& c) {
+#ifdef __HIP_DEVICE_COMPILE__
+  sincos(x, &s, &c);
+#else
+  s = sin(x);
+  c = cos(x);
+#endif
+}
+// The unit vector of the angles phi and theta.
+__device__ inline V3 unitVector(double phi, double theta) {
+  double sp, cp, st, ct;
+  sinCos(phi, sp, cp);
+  sinCos(theta, st, ct);
+  return mk(cp * st, sp * st, ct);
+}
 __device__ inline double divBy6(double a) { return divBy(a, 6.0, 1.0 / 6.0); }
 
 constexpr int kCellValues = 24;

@@ -234,10 +234,15 @@ KF_HD V3 localToGlobal(const DevSurface& s, double l0, double l1) {
   if (s.type == ACTS_KF_SURFACE_CYLINDER) {
     const double r = s.b0;
     const double phi = l0 / r;
-    return toGlobal(s.R, s.t, mk(r * cos(phi), r * sin(phi), l1));
+    double sp, cp;
+    sinCos(phi, sp, cp);
+    return toGlobal(s.R, s.t, mk(r * cp, r * sp, l1));
   }
-  if (s.type == ACTS_KF_SURFACE_DISC)
-    return toGlobal2(s.R, s.t, l0 * cos(l1), l0 * sin(l1));
+  if (s.type == ACTS_KF_SURFACE_DISC) {
+    double sp, cp;
+    sinCos(l1, sp, cp);
+    return toGlobal2(s.R, s.t, l0 * cp, l0 * sp);
+  }
   return toGlobal2(s.R, s.t, l0, l1);
 }
 
@@ -283,7 +288,8 @@ KF_HD void positionJacobians(const DevSurface& s, const V3& pos, double b2f[6], 
     const V3 posLoc = toLocal(s, pos);
     const double lr = perp(posLoc);
     const double lphi = atan2(posLoc.y, posLoc.x);
-    const double lc = cos(lphi), ls = sin(lphi);
+    double lc, ls;
+    sinCos(lphi, ls, lc);
     for (int i = 0; i < 3; ++i) {
       const double lx = s.R[3 * i + 0], ly = s.R[3 * i + 1];
       const double c0 = lc * lx + ls * ly;

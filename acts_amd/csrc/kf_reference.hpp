@@ -190,8 +190,7 @@ __device__ inline int lineBoundState(const Track& T, const LineRef& L, double to
 template <bool Sympy = false>
 __device__ inline void initializeFromBound(Track& T, const DevSurface& s, const double p[6],
                                            const double c[21], const DevOpts& o) {
-  const double sinTheta = sin(p[3]);
-  T.dir = mk(cos(p[2]) * sinTheta, sin(p[2]) * sinTheta, cos(p[3]));
+  T.dir = unitVector(p[2], p[3]);
   T.pos = localToGlobal(s, p[0], p[1]);
   T.time = p[5];
   T.qop = p[4];
@@ -265,8 +264,7 @@ __device__ inline int extrapolateTrack(int64_t q, const DevScratch& sc, const do
   // the straight-line distance from a state's smoothed parameters
   auto distanceFrom = [&](int k, const double* p, double& path) -> bool {
     const DevSurface& s = geo[si(sc, k, kISurf, q)];
-    const double sinTheta = sin(p[3]);
-    const V3 dir = mk(cos(p[2]) * sinTheta, sin(p[2]) * sinTheta, cos(p[3]));
+    const V3 dir = unitVector(p[2], p[3]);
     const V3 pos = localToGlobal(s, p[0], p[1]);
     return lineIntersect(L, pos, dir, kOnSurfaceTolerance, path) != kUnreachable;
   };

@@ -70,8 +70,8 @@ __device__ inline int laneInitReverse(Lane& L, const int64_t q, const int64_t t,
   L.noTransport = false;
   L.replaying = false;
   L.noSkip = false;
-  L.nUnique = uniqueMeasurementSurfaces(in, L.m0, L.nMeas);
-  L.mNext = 0;
+  L.nUnique = uniqueMeasurementSurfaces(in, L.m0, L.nMeas, L.measSet);
+  L.mNext = L.nMeas;
   a.rv.reached[q] = 0;
   const int lastMeas = sc.track[3 * sc.stride + q];
   const int surf = si(sc, lastMeas, kISurf, q);
