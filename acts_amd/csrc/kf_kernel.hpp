@@ -662,6 +662,50 @@ __device__ inline void storeSym(double* dst, const double* p) {
     for (int j = 0; j < 6; ++j) dst[6 * i + j] = p[sym(i, j)];
 }
 
+// A state's smoothed parameters and covariance as they stand in the outputs,
+// for each lane of a wavefront.
+struct SmoothedRows {
+  static constexpr int kCov = 36, kRow = 42;
+  alignas(16) double v[64 * kRow];
+  int64_t slot[64];  // output slot of the lane's row, -1: no row
+};
+
+// Writes the rows of a wavefront to the outputs.  A lane's row is 288 + 48
+// contiguous bytes, another track's rows are kilobytes away: written from the
+// lane's registers every store touches 64 places, and the stores' address
+// processing held the smoother up (a third of its wavefronts' cycles); here 18
+// lanes write a row together, 3 rows a store.
+__device__ inline void storeRows(const SmoothedRows& s, const DevOut& out) {
+  using Pair = double __attribute__((ext_vector_type(2)));
+  struct __attribute__((packed, aligned(8))) Pair8 {
+    Pair v;
+  };
+  constexpr int kPairs = SmoothedRows::kCov / 2;
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  if (out.smoothedCov) {
+    const int sub = lane / kPairs, off = lane % kPairs;
+#pragma unroll
+    for (int r = 0; r < 64; r += 3) {
+      const int row = r + sub;
+      if (sub < 3 && row < 64) {
+        const int64_t slot = s.slot[row];
+        const Pair x = *reinterpret_cast<const Pair*>(s.v + SmoothedRows::kRow * row + 2 * off);
+        if (slot >= 0) reinterpret_cast<Pair8*>(out.smoothedCov + 36 * slot)[off].v = x;
+      }
+    }
+  }
+  if (out.smoothed) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int c = 64 * i + lane, row = c / 3, off = c % 3;
+      const int64_t slot = s.slot[row];
+      const Pair x = *reinterpret_cast<const Pair*>(s.v + SmoothedRows::kRow * row +
+                                                    SmoothedRows::kCov + 2 * off);
+      if (slot >= 0) reinterpret_cast<Pair8*>(out.smoothed + 6 * slot)[off].v = x;
+    }
+  }
+}
+
 // GainMatrixSmoother::operator() from the tip backwards, the track summary
 // (calculateTrackQuantities) and the per-state outputs.
 // `valid` is false for the padding lanes of the last wavefront: they take
@@ -892,7 +936,9 @@ __device__ inline void mbfUpdate(int64_t q, int64_t t, int k, uint32_t flags, co
 template <bool Mbf>
 __device__ inline void smoothTrack(const int64_t q, const int64_t t, const bool valid,
                                    const DevBatch& in,
-                                   const DevOut& out, const DevScratch& sc, const bool rev) {
+                                   const DevOut& out, const DevScratch& sc, const bool rev,
+                                   const bool shareRows, SmoothedRows& rows) {
+  const int lane = static_cast<int>(threadIdx.x) & 63;
   int status = valid ? sc.track[q] : 0;
   const int tip = (!valid || status) ? -1 : sc.track[sc.stride + q];
   // with a reference surface: keep the smoothed first and last measurement
@@ -916,8 +962,9 @@ __device__ inline void smoothTrack(const int64_t q, const int64_t t, const bool 
     for (int i = 0; i < 6; ++i) l[i] = 0.0;
   }
   bool active = tip >= 0;
-  for (int k = kTop; k >= 0; --k) {
-    if (!active || k > tip) continue;
+  // One state of the lane; false: no row to write.
+  auto state = [&](int k) -> bool {
+    if (!active || k > tip) return false;
     double xf[6], Cf[21], xs[6], Cs[21], CsFull[36];
 #pragma unroll
     for (int i = 0; i < 6; ++i) xf[i] = sd(sc, k, kFilt + i, q);
@@ -954,7 +1001,7 @@ __device__ inline void smoothTrack(const int64_t q, const int64_t t, const bool 
       if (r) {
         status = r;
         active = false;
-        continue;
+        return false;
       }
     }
     if (!rev && (k == firstMeas || k == lastMeas)) {
@@ -980,13 +1027,25 @@ __device__ inline void smoothTrack(const int64_t q, const int64_t t, const bool 
       ndf += in.measDims ? in.measDims[in.measOff[t] + si(sc, k, kIMeas, q)] : 2;
     }
     const int64_t slot = base + k;
-    if (out.smoothed)
-      for (int i = 0; i < 6; ++i) out.smoothed[6 * slot + i] = xs[i];
-    if (out.smoothedCov) {
+    if (shareRows) {
+      double* row = rows.v + SmoothedRows::kRow * lane;
       if constexpr (Mbf) {
-        for (int i = 0; i < 36; ++i) out.smoothedCov[36 * slot + i] = CsFull[i];
+#pragma unroll
+        for (int i = 0; i < 36; ++i) row[i] = CsFull[i];
       } else {
-        storeSym(out.smoothedCov + 36 * slot, Cs);
+        storeSym(row, Cs);
+      }
+#pragma unroll
+      for (int i = 0; i < 6; ++i) row[SmoothedRows::kCov + i] = xs[i];
+    } else {
+      if (out.smoothed)
+        for (int i = 0; i < 6; ++i) out.smoothed[6 * slot + i] = xs[i];
+      if (out.smoothedCov) {
+        if constexpr (Mbf) {
+          for (int i = 0; i < 36; ++i) out.smoothedCov[36 * slot + i] = CsFull[i];
+        } else {
+          storeSym(out.smoothedCov + 36 * slot, Cs);
+        }
       }
     }
     if (out.filtered)
@@ -1016,6 +1075,16 @@ __device__ inline void smoothTrack(const int64_t q, const int64_t t, const bool 
       for (int i = 0; i < 6; ++i) xsN[i] = xs[i];
 #pragma unroll
       for (int i = 0; i < 21; ++i) CsN[i] = Cs[i];
+    }
+    return true;
+  };
+  for (int k = kTop; k >= 0; --k) {
+    const bool row = state(k);
+    if (shareRows) {
+      rows.slot[lane] = row ? base + k : -1;
+      __syncthreads();
+      storeRows(rows, out);
+      __syncthreads();
     }
   }
   if (!valid) return;
