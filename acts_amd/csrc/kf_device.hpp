@@ -230,17 +230,29 @@ KF_HD bool globalToLocal(const DevSurface& s, const V3& pos,
   return true;
 }
 
+// (TwoReductions: sine and cosine by themselves.  The track-state table's
+// kernel keeps 168 registers with them, three wavefronts per SIMD, and 212
+// with one reduction: 0.567 against 0.576 ms per 100 000 endcap tracks.)
+template <bool TwoReductions = false>
 KF_HD V3 localToGlobal(const DevSurface& s, double l0, double l1) {
+  auto angle = [](double x, double& sn, double& cs) {
+    if (TwoReductions) {
+      sn = sin(x);
+      cs = cos(x);
+    } else {
+      sinCos(x, sn, cs);
+    }
+  };
   if (s.type == ACTS_KF_SURFACE_CYLINDER) {
     const double r = s.b0;
     const double phi = l0 / r;
     double sp, cp;
-    sinCos(phi, sp, cp);
+    angle(phi, sp, cp);
     return toGlobal(s.R, s.t, mk(r * cp, r * sp, l1));
   }
   if (s.type == ACTS_KF_SURFACE_DISC) {
     double sp, cp;
-    sinCos(l1, sp, cp);
+    angle(l1, sp, cp);
     return toGlobal2(s.R, s.t, l0 * cp, l0 * sp);
   }
   return toGlobal2(s.R, s.t, l0, l1);

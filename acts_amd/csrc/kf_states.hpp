@@ -133,7 +133,7 @@ KF_HD void paramColumns(const DevSurface& s, const double* x, const double* diag
   sincos(x[2], &sphi, &cphi);
   sincos(x[3], &sth, &cth);
   const V3 dir = mk(cphi * sth, sphi * sth, cth);
-  const V3 pos = localToGlobal(s, x[0], x[1]);
+  const V3 pos = localToGlobal<true>(s, x[0], x[1]);
   const double p = fabs(1 / x[4]);
   put(base + 24, clampF(pos.x));
   put(base + 25, clampF(pos.y));
@@ -227,7 +227,7 @@ __device__ inline void trackStateRow(const TsArgs& a, int64_t slot) {
       sincos(truth[2], &sphi, &cphi);
       sincos(truth[3], &sth, &cth);
       const V3 tdir = mk(cphi * sth, sphi * sth, cth);
-      const V3 tpos = localToGlobal(s, truth[0], truth[1]);
+      const V3 tpos = localToGlobal<true>(s, truth[0], truth[1]);
       put(ACTS_KF_TS_T_X + 0, clampF(tpos.x));
       put(ACTS_KF_TS_T_X + 1, clampF(tpos.y));
       put(ACTS_KF_TS_T_X + 2, clampF(tpos.z));
@@ -248,7 +248,7 @@ __device__ inline void trackStateRow(const TsArgs& a, int64_t slot) {
       // (0 where not measured)
       const double l0 = (ma == 0) ? m[0] : ((mdim == 2 && mb == 0) ? m[1] : 0.0);
       const double l1 = (ma == 1) ? m[0] : ((mdim == 2 && mb == 1) ? m[1] : 0.0);
-      const V3 g = localToGlobal(s, l0, l1);
+      const V3 g = localToGlobal<true>(s, l0, l1);
       put(ACTS_KF_TS_L_X_HIT + 0, clampF(l0));
       put(ACTS_KF_TS_L_X_HIT + 1, clampF(l1));
       put(ACTS_KF_TS_L_X_HIT + 2, clampF(g.x));
