@@ -553,8 +553,8 @@ struct MapField {
         for (int j = 0; j < kCellValues; ++j) v[j] = c.v[j * kCellCacheStride];
       }
       if (!hit) {
-        const double* q = static_cast<const double*>(
-            __builtin_assume_aligned(F.cells + static_cast<int64_t>(kCellDoubles) * cell, 64));
+        const auto q = (GlobalPtr<double>)__builtin_assume_aligned(
+            F.cells + static_cast<int64_t>(kCellDoubles) * cell, 64);
 #pragma unroll
         for (int j = 0; j < kCellValues; ++j) v[j] = q[j];
         if (c.idx) {

@@ -112,7 +112,10 @@ struct FwdArgs {
 // steps (the empty asm makes their values ones that cannot be read again).
 // Left to the compiler each is read where it is used, 7 reads a step in a
 // uniform field and 35 in a map, and a wavefront that is alone on its SIMD
-// stands still for every one of them.
+// stands still for every one of them.  (A map's are more than fit: some are
+// fetched back from lanes of vector registers.)  The map's pointers no longer
+// say that they point to global memory: what loads through them says so itself
+// (GlobalPtr).
 struct StepArgs {
   DevOpts o;
   DevField F;

@@ -103,8 +103,8 @@ struct MapFieldF {
         for (int j = 0; j < kCellValues; ++j) v[j] = c.vf[j * kCellCacheStride];
       }
       if (!hit) {
-        const float* q = static_cast<const float*>(
-            __builtin_assume_aligned(F.cellsF + static_cast<int64_t>(kCellFloats) * cell, 128));
+        const auto q = (GlobalPtr<float>)__builtin_assume_aligned(
+            F.cellsF + static_cast<int64_t>(kCellFloats) * cell, 128);
 #pragma unroll
         for (int j = 0; j < kCellValues; ++j) v[j] = q[j];
         if (c.idx) {
