@@ -23,7 +23,7 @@ OBJECTS = [("kf_capi.hip", []), ("generator.hip", [])] + [
     for m in (0, 1) for s in (0, 1) for n in (0, 1) for f in (0, 1)]
 HEADERS = ["kf_common.hpp", "kf_device.hpp", "kf_mixed.hpp", "kf_fit.hpp", "kf_kernel.hpp",
            "kf_reference.hpp", "kf_reverse.hpp", "kf_forward.hpp", "kf_states.hpp",
-           "kf_host_copy.hpp", "kf_field_host.hpp"]
+           "kf_host_copy.hpp", "kf_queue.hpp", "kf_field_host.hpp"]
 
 # -ffp-contract=off: the FP64 fit keeps the reference's separate multiply and
 # add roundings (x86-64 without -march has no FMA), so every decision of the

@@ -16,6 +16,7 @@
 #include "kf_reference.hpp"
 #include "kf_forward.hpp"
 #include "kf_host_copy.hpp"
+#include "kf_queue.hpp"
 #include "kf_states.hpp"
 
 using namespace kf;
@@ -120,26 +121,6 @@ __global__ __launch_bounds__(kBlock) void referenceKernel(DevOut out, DevScratch
 __global__ void zeroKernel(int32_t* p, int32_t count) {
   const int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
   if (i < count) p[i] = 0;
-}
-
-// Queue place of sorted place i: the nSeam first tracks (the ones that may
-// become loopers) `spacing` places apart over the first `window` places, the
-// others between them.  In one block they filled the first wavefronts, where
-// loopers with different targets and step lengths took each other's steps
-// too (a step of several in the field map 3.2 to 3.8 against 2.4 thousand
-// x 4 cycles of one alone), which sets the length of a fit that is over
-// before its loopers: forward kernel of 5 000 field-map tracks 4.6 -> 4.2
-// ms, 100 000 7.1 -> 5.6, 200 000 7.2 -> 6.0.  A larger batch keeps the
-// block (window 1): few wavefronts then stay behind in quarantine with
-// their loopers while the others fit the rest (500 000: 6.7, spread 7.7 ms).
-constexpr int64_t kSpreadBatch = 4;  // batches, in resident lanes, to spread
-__device__ inline int32_t spreadPlace(int32_t i, int32_t nSeam, int32_t window) {
-  const int32_t spacing = nSeam > 0 ? min(64, window / nSeam) : 0;
-  if (spacing <= 1) return i;
-  const int32_t j = i - nSeam;
-  if (j < 0) return i * spacing;
-  if (j < nSeam * (spacing - 1)) return j / (spacing - 1) * spacing + 1 + j % (spacing - 1);
-  return i;
 }
 
 // Counting sort of the tracks by sequence length, longest first.
@@ -359,7 +340,7 @@ constexpr int kSmallSort = 4096;
 constexpr int kSmallSortThreads = 1024;
 __global__ __launch_bounds__(kSmallSortThreads) void smallSortKernel(QueueKeyArgs k, int32_t n,
                                                                      int32_t nKeys, int32_t* perm,
-                                                                     int32_t* queue, int32_t window) {
+                                                                     int32_t* queue, Spread spread) {
   __shared__ int32_t key[kSmallSort];  // first the seam marks
   __shared__ int32_t h[kMaxKeys];
   __shared__ int32_t waves[kSmallSortThreads / 64];
@@ -396,14 +377,14 @@ __global__ __launch_bounds__(kSmallSortThreads) void smallSortKernel(QueueKeyArg
   const int32_t nSeam = h[nKeys - 2];
   __syncthreads();
   for (int t = tid; t < n; t += kSmallSortThreads)
-    perm[spreadPlace(atomicAdd(&h[key[t]], 1), nSeam, window)] = t;
+    perm[spreadPlace(atomicAdd(&h[key[t]], 1), nSeam, spread)] = t;
 }
 
 __global__ __launch_bounds__(kSortBlock) void keyScatterKernel(const int32_t* keys, int64_t n,
                                                                int32_t nKeys,
                                                                const int32_t* blockOffset,
                                                                int32_t* perm, int32_t* queue,
-                                                               int32_t window) {
+                                                               Spread spread) {
   const int32_t nSeam = blockOffset[histIndex(nKeys - 2, nKeys, 0, gridDim.x)];
   __shared__ int32_t h[kMaxKeys];
   if (blockIdx.x == 0 && threadIdx.x == 0) *queue = 0;
@@ -415,7 +396,7 @@ __global__ __launch_bounds__(kSortBlock) void keyScatterKernel(const int32_t* ke
     const int32_t key = keys[t];
     const int32_t rank = atomicAdd(&h[key], 1);
     perm[spreadPlace(blockOffset[histIndex(key, nKeys, blockIdx.x, gridDim.x)] + rank, nSeam,
-                     window)] = static_cast<int32_t>(t);
+                     spread)] = static_cast<int32_t>(t);
   }
 }
 
@@ -1204,12 +1185,11 @@ static int launchFit(acts_kf_ctx* c, const acts_kf_batch_in* in,
     qk.geo = c->geo;
     qk.nSurfaces = c->nSurfaces;
     qk.maxLen = states;
-    const int64_t lanes = c->residentWaves * kBlock;
-    const int32_t window =
-        n <= kSpreadBatch * lanes ? static_cast<int32_t>(std::min<int64_t>(n, lanes)) : 1;
+    const Spread spread = spreadOf(n, c->residentWaves * kBlock,
+                                   c->opts.navigator != ACTS_KF_NAVIGATOR_DIRECT);
     if (n <= kSmallSort) {
       hipLaunchKernelGGL(smallSortKernel, dim3(1), dim3(kSmallSortThreads), 0, stream, qk,
-                         static_cast<int32_t>(n), nKeys, perm, ws.queue, window);
+                         static_cast<int32_t>(n), nKeys, perm, ws.queue, spread);
     } else {
       const unsigned nb = static_cast<unsigned>(sortBlocks);
       const unsigned nbKey = static_cast<unsigned>((n + kSortBlock - 1) / kSortBlock);
@@ -1227,7 +1207,7 @@ static int launchFit(acts_kf_ctx* c, const acts_kf_batch_in* in,
       hipLaunchKernelGGL(chunkScanKernel, dim3(chunks), dim3(kScanThreads), 0, stream, hist, count,
                          sums);
       hipLaunchKernelGGL(keyScatterKernel, dim3(nb), dim3(kSortBlock), 0, stream, keys, n,
-                         nKeys, hist, perm, ws.queue, window);
+                         nKeys, hist, perm, ws.queue, spread);
     }
   } else {
     hipLaunchKernelGGL(zeroKernel, dim3(1), dim3(64), 0, stream, ws.queue, 1);
