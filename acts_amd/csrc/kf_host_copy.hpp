@@ -17,7 +17,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 
 namespace kf {
@@ -171,8 +171,8 @@ class HostCopy {
     for (int t = 1; t < threads; ++t) {
       try {
         pool[t] = std::thread(work, t);
-      } catch (const std::system_error&) {
-        work(t);  // no thread to be had: its share is done here
+      } catch (const std::exception&) {
+        work(t);  // no thread, or no memory for one: its share is done here
       }
     }
     work(0);

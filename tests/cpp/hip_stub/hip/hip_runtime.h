@@ -4,6 +4,8 @@
 
 #include <cmath>
 
+#include "hip_runtime_api.h"
+
 #define __host__
 #define __device__
 
