@@ -41,11 +41,16 @@ SPACE = {
     "sched_inner_steps": [8, 16, 32, 64, 128],
     "sched_wait_64ths": [16, 32, 48, 64],
     "length_sorted": [1, 0, 2, 3],
-    "sched_quarantine_steps": [0, 100, 200, 400, -1],
+    "sched_quarantine_steps": [0, 100, 400, -1],  # 0: the library's 200
     "sched_transport_skip_steps": [0, 64, -1],
 }
 DEFAULTS = {"sched_inner_steps": 16, "sched_wait_64ths": 64, "length_sorted": 1,
             "sched_quarantine_steps": 0, "sched_transport_skip_steps": 0}
+# What the knobs' values mean, as part of a cache entry's key: raised when a
+# meaning changes.  2: 0 is the library's default for the quarantine and the
+# transport skip, not "off" (that is -1), so that settings measured with 0 as
+# "off" are not applied as 200.
+KNOBS_VERSION = 2
 
 
 def coordinate_descent(evaluate: Callable[[dict], float], space=SPACE, start=None,
@@ -82,7 +87,7 @@ def signature(events, field, options, device_name: str = "") -> str:
     return json.dumps({"n": n_bucket, "max_len": int(lens.max() if n else 0),
                        "mean_len": round(float(lens.mean()) if n else 0.0, 1),
                        "field": type(field).__name__, "precision": int(options.precision),
-                       "device": device_name}, sort_keys=True)
+                       "device": device_name, "knobs": KNOBS_VERSION}, sort_keys=True)
 
 
 def default_cache_path() -> str:

@@ -249,8 +249,8 @@ typedef struct acts_kf_options {
    * sched_wait_64ths  the surface update runs early once this many 64ths of
    *                   the busy lanes of a wavefront wait (0 = 64: all);
    * sched_quarantine_steps  a wavefront takes no new tracks while one of its
-   *                   tracks has run more than this many steps (0 = 200,
-   *                   negative = off).                                      */
+   *                   tracks has run more than this many steps (0 = the
+   *                   default, 200; negative = off; 0 once meant off).      */
   int32_t length_sorted;
   int32_t sched_inner_steps;
   int32_t sched_wait_64ths;
@@ -267,12 +267,12 @@ typedef struct acts_kf_options {
    * surface after all, it goes back to the saved state and repeats those
    * steps with the transport, so the results do not depend on it (a track
    * that never reaches another surface, e.g. a looper that ends at
-   * max_steps, uses no transport).  0 = the default: 200 steps in a uniform
-   * field; off in a field map, where loopers come back to a surface, repeat
-   * the skipped steps and lose more than they save.  Negative = off; always
-   * off with the layer navigator.  The saved states take up to 52 MB of
-   * device memory, grown with the batch; where they cannot be allocated the
-   * fit runs without.  No reference counterpart.                            */
+   * max_steps, uses no transport).  0 = the default (it once meant off): 200
+   * steps in a uniform field; off in a field map, where loopers come back to
+   * a surface, repeat the skipped steps and lose more than they save.
+   * Negative = off; always off with the layer navigator.  The saved states
+   * take up to 52 MB of device memory, grown with the batch; where they cannot
+   * be allocated the fit runs without.  No reference counterpart.           */
   int32_t sched_transport_skip_steps;
   /* ACTS_KF_NAVIGATOR_* (default DIRECT)                                    */
   int32_t navigator;
