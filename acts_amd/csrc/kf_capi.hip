@@ -332,10 +332,10 @@ __global__ __launch_bounds__(kScanThreads) void chunkScanKernel(int32_t* a, int6
 }
 
 // The whole sort of a small batch in one workgroup and one launch: keys,
-// histogram, scan and scatter in LDS, and the queue counter.  The six
-// launches of the general sort took ~45 us, of which 9 in the scan of the
-// chunk sums, against ~15 for this at its largest batch, where one CU's
-// reading of the measurements begins to show.
+// histogram, scan and scatter in LDS, and the queue counter.  The general sort
+// was six launches then, and one more for the counter: ~45 us, of which 9 in
+// the scan of the chunk sums, against ~15 for this at its largest batch, where
+// one CU's reading of the measurements begins to show.
 constexpr int kSmallSort = 4096;
 constexpr int kSmallSortThreads = 1024;
 __global__ __launch_bounds__(kSmallSortThreads) void smallSortKernel(QueueKeyArgs k, int32_t n,

@@ -264,18 +264,20 @@ struct DevField {
 // the second gives the correctly rounded quotient (Markstein's theorem,
 // IBM J. Res. Dev. 34 (1990) 111; Muller et al., Handbook of Floating-Point
 // Arithmetic, 2018, sec. 4.9), i.e. exactly a / b, for normal b, y and a
-// quotient far from overflow and underflow.  Five full-rate operations in
-// place of the division's scale, reciprocal, refinement and fix-up sequence
-// (2 % off the FP64 field-map forward kernel; the same for the FP32 map's
-// divisions measured 4 % slower than the division, so it divides).
+// quotient (and its residual) far from overflow and underflow.  Five full-rate
+// operations in place of the division's scale, reciprocal, refinement and
+// fix-up sequence (2 % off the FP64 field-map forward kernel; the FP32 map's
+// lookups do the same, divRecipF).
 KF_HD double divRecip(double a, double b, double y) {
   double q = a * y;
   q = fma(fma(-q, b, a), y, q);
   return fma(fma(-q, b, a), y, q);
 }
 
-// a / b from y = RN(1/b) in every case: the fix-up instruction gives the
-// results of the special operands (zeros with their sign, infinities, NaN).
+// a / b from y = RN(1/b) on divRecip's domain and for the special operands,
+// whose results the fix-up instruction gives (zeros with their sign,
+// infinities, NaN).  Not for subnormal b or 1/b or a quotient near underflow,
+// which the norms of directions, step lengths and momenta here do not reach.
 __device__ inline double divBy(double a, double b, double y) {
   return __builtin_amdgcn_div_fixup(divRecip(a, b, y), b, a);
 }

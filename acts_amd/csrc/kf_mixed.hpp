@@ -201,7 +201,7 @@ __device__ inline int rkStepMixed(Track& T, const Field& field, const DevOpts& o
   }
   if (status) return status;
 
-  // time and its derivatives in double (as rkTime): the time is not
+  // time and its derivatives in double (as rkApply): the time is not
   // measured, so its smoothed value is set by these jacobian entries through
   // the ill-conditioned RTS gain, which magnifies float rounding to ~1e-5
   const float m = o.mass;

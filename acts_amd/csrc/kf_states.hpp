@@ -2,9 +2,12 @@
 // (Examples/Io/Root/src/RootTrackStatesWriter.cpp:364-735) computed on the
 // device from a fitted batch, one thread per state slot, column-major
 // float output so that every column store of a wavefront is one coalesced
-// 256-byte line.  The work per state is ~1.1 KB of reads (three parameter
-// vectors and covariances, the measurement, the truth) and 0.6 KB of
-// writes against ~600 FLOP: the kernel is HBM-bound.
+// 256-byte line.  The kernel is HBM-bound: ~1.1 KB read (three parameter
+// vectors and covariances, of which the diagonals lie in every cache line, the
+// measurement, the truth) and 0.6 KB written per state, 2.55 GB for 100 000
+// endcap tracks, take 495 of its 566 us at the 5.15 TB/s of a large copy; the
+// FP64 work (~5 k lane instructions per state) fills 14 % of a wavefront's time
+// at three wavefronts per SIMD.
 #pragma once
 
 #include <cfloat>
@@ -159,9 +162,7 @@ constexpr int kTsBlock = 256;
 // One row of the table, for slot `slot`: everything RootTrackStatesWriter
 // derives from one track state (the body of its state loop,
 // RootTrackStatesWriter.cpp:364-735).  The row is computed in FP64 and
-// stored as float: the cost is the FP64 transcendental and division work
-// of four parameter sets (~5 k lane instructions per state), not the
-// 1.8 KB it moves.
+// stored as float.
 // Sub: the batch has measurement subspaces (dimension and indices read per
 // measurement); otherwise every measurement is 2D on (loc0, loc1), known at
 // compile time.

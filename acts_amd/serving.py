@@ -54,10 +54,11 @@ class ServingConfig:
     slots: int = 3                   # fitter contexts: most batches in flight
     hbm_budget_bytes: float = 32e9   # device memory of all batches in flight
     # tracks per batch: a batch's forward kernel lasts as long as its slowest
-    # track (a looper that ends at max_steps: ~9 ms in the field map whether
-    # the batch holds 48 000 tracks or 500 000), so large batches amortise
-    # it; measured saturated capacity in the field map with 3 slots: 6.9 M
-    # tracks/s at 60 000, 8.1 M at 150 000, 13.8 M at 300 000
+    # track (a looper that ends at max_steps: ~5 ms in the field map whether
+    # the batch holds 5 000 tracks or 300 000), so large batches amortise
+    # it; measured saturated capacity in the field map with 3 slots, when that
+    # was ~9 ms: 6.9 M tracks/s at 60 000, 8.1 M at 150 000, 13.8 M at 300 000
+    # (now 15.6 M)
     max_batch_tracks: int = 300000
     seed: int = 1
     keep_results: bool = False       # keep every event's results (tests)

@@ -271,7 +271,7 @@ typedef struct acts_kf_options {
    * steps in a uniform field; off in a field map, where loopers come back to
    * a surface, repeat the skipped steps and lose more than they save.
    * Negative = off; always off with the layer navigator.  The saved states
-   * take up to 52 MB of device memory, grown with the batch; where they cannot
+   * take up to 54 MB of device memory, grown with the batch; where they cannot
    * be allocated the fit runs without.  No reference counterpart.           */
   int32_t sched_transport_skip_steps;
   /* ACTS_KF_NAVIGATOR_* (default DIRECT)                                    */
@@ -394,9 +394,15 @@ int acts_kf_create(const acts_kf_surface* surfaces, int32_t n_surfaces,
                    const acts_kf_field* field, const acts_kf_options* options,
                    int32_t device, acts_kf_ctx** out_ctx);
 
-/* Fit a batch whose buffers (in and out) are host memory.  Asynchronous on
- * `stream` (a hipStream_t, NULL = the context's own stream); results are in
- * the output buffers after acts_kf_sync.  seq_offsets and meas_offsets must
+/* Fit a batch whose buffers (in and out) are host memory, on `stream` (a
+ * hipStream_t, NULL = the context's own stream); results are in the output
+ * buffers after acts_kf_sync.  With pinned outputs the call is asynchronous
+ * (pinned inputs then have to stay until acts_kf_sync); with any pageable
+ * output it returns when the fit and its copies are done.  Pageable arrays go
+ * through pinned memory of the context (up to 32 MiB, kept until
+ * acts_kf_destroy), more than 2 MiB of them in each direction with the help
+ * of up to 7 threads that end before the call returns; while `stream` is being
+ * captured they take the runtime's copies.  seq_offsets and meas_offsets must
  * start at 0 and never decrease (ACTS_KF_ERR_INVALID_ARGUMENT otherwise).  Replaces one call of
  * KalmanFitter::fit (KalmanFitter.hpp:721-731, the DirectNavigator overload
  * with the surface sequence) per track of the batch, as issued by
